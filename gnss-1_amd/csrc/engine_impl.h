@@ -273,32 +273,7 @@ class Engine : public EngineBase {
 
   void stats(gnss_stats_out* o, double* yprof, double* spectrum) override {
     need_k();
-    const int nb = n_bins();
-    stats_kernels(d_part_, d_spec_, d_prof_, d_cmax_);
-    std::vector<double> part((size_t)nx_ * SPEC_NQ), spec((size_t)nx_ * (1 + S_) * nb),
-        prof((size_t)(7 + 3 * S_) * ny_), cm((size_t)2 * ny_);
-    GNSS_HIP(hipMemcpyAsync(part.data(), d_part_, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s_));
-    GNSS_HIP(hipMemcpyAsync(spec.data(), d_spec_, sizeof(double) * spec.size(), hipMemcpyDeviceToHost, s_));
-    GNSS_HIP(hipMemcpyAsync(prof.data(), d_prof_, sizeof(double) * prof.size(), hipMemcpyDeviceToHost, s_));
-    GNSS_HIP(hipMemcpyAsync(cm.data(), d_cmax_, sizeof(double) * cm.size(), hipMemcpyDeviceToHost, s_));
-    sync();
-    double sum[SPEC_NQ + 2] = {0};
-    for (int x = 0; x < nx_; ++x)
-      for (int qq = 0; qq < SPEC_NQ; ++qq) sum[qq] += part[(size_t)x * SPEC_NQ + qq];
-    for (int y = 0; y < ny_; ++y) {
-      sum[SPEC_NQ] = std::max(sum[SPEC_NQ], cm[2 * y]);
-      sum[SPEC_NQ + 1] = std::max(sum[SPEC_NQ + 1], cm[2 * y + 1]);
-    }
-    stats_finish(sum, o);
-    if (yprof) memcpy(yprof, prof.data(), sizeof(double) * prof.size());
-    if (spectrum) {
-      for (int s = 0; s <= S_; ++s)
-        for (int b = 0; b < nb; ++b) {
-          double acc = 0;
-          for (int x = 0; x < nx_; ++x) acc += spec[((size_t)x * (1 + S_) + s) * nb + b];
-          spectrum[(size_t)s * nb + b] = acc;
-        }
-    }
+    stats_run(d_part_, d_spec_, d_prof_, d_cmax_, d_fin_, o, yprof, spectrum);
   }
 
   // Scratch layout of stats_noalloc, regions 256-byte aligned: per-plane spectral sums, per-plane
@@ -322,59 +297,82 @@ class Engine : public EngineBase {
   size_t stats_scratch_doubles() const override { return stat_scratch_layout().total; }
 
   // Every partial the kernels read is written earlier in the same call, so the scratch needs no
-  // clearing; the sums over planes run on the device in the order stats() sums them on the host.
+  // clearing.
   void stats_noalloc(double* scratch, gnss_stats_out* o, double* yprof, double* spectrum) override {
     need_k();
-    const int nb = n_bins();
     const StatScratch l = stat_scratch_layout();
-    double* fin = scratch + l.fin;
     pause_timer_ = true;
     try {
-      stats_kernels(scratch + l.part, scratch + l.spec, scratch + l.prof, scratch + l.cmax);
+      stats_run(scratch + l.part, scratch + l.spec, scratch + l.prof, scratch + l.cmax, scratch + l.fin, o, yprof,
+                spectrum);
     } catch (...) {
       pause_timer_ = false;
       throw;
     }
     pause_timer_ = false;
-    hipLaunchKernelGGL(k_stats_reduce, dim3(1), dim3(STAT_THREADS), 0, s_, scratch + l.part, scratch + l.spec,
-                       scratch + l.cmax, nx_, ny_, (1 + S_) * nb, fin);
-    check_launch("k_stats_reduce");
+  }
+
+  // The statistics with their partial sums in the given device memory.  The sums over planes run on
+  // the device, so that only the results cross to the host (the shell partials of every plane are
+  // nx times as many: 3.6 MB at 512^3).
+  void stats_run(double* part, double* spec, double* prof, double* cmax, double* fin, gnss_stats_out* o, double* yprof,
+                 double* spectrum) {
+    const int nspec = spectrum ? (1 + S_) * n_bins() : 0;
+    stats_kernels(part, spectrum ? spec : nullptr, prof, cmax);
+    // reported as the spectrum's time: its sums over the planes are nearly all of this kernel's
+    timed("k_spectrum", (double)nx_ * (SPEC_NQ + nspec) * sizeof(double), [&] {
+      hipLaunchKernelGGL(k_stats_reduce, dim3((unsigned)cdiv(SPEC_NQ + 2 + nspec, 64)), dim3(64), 0, s_, part, spec,
+                         cmax, nx_, ny_, nspec, fin);
+    });
     double sum[SPEC_NQ + 2];
     GNSS_HIP(hipMemcpyAsync(sum, fin, sizeof(sum), hipMemcpyDeviceToHost, s_));
     if (yprof)
-      GNSS_HIP(hipMemcpyAsync(yprof, scratch + l.prof, sizeof(double) * (7 + 3 * S_) * ny_, hipMemcpyDeviceToHost, s_));
+      GNSS_HIP(hipMemcpyAsync(yprof, prof, sizeof(double) * (7 + 3 * S_) * ny_, hipMemcpyDeviceToHost, s_));
     if (spectrum)
-      GNSS_HIP(hipMemcpyAsync(spectrum, fin + SPEC_NQ + 2, sizeof(double) * (1 + S_) * nb, hipMemcpyDeviceToHost, s_));
+      GNSS_HIP(hipMemcpyAsync(spectrum, fin + SPEC_NQ + 2, sizeof(double) * nspec, hipMemcpyDeviceToHost, s_));
     sync();
     stats_finish(sum, o);
   }
 
-  // Statistics kernels: spectral sums and shell sums per kx plane, the physical fields, then the
-  // planar averages and maxima per y.
+  // Statistics kernels: spectral sums (and shell sums, unless spec is null) per kx plane, the physical
+  // fields, then the planar averages and maxima per y.
   void stats_kernels(double* part, double* spec, double* prof, double* cmax) {
     const double nn = (double)nx_ * ny_ * nz_;
     const double inn2 = 1.0 / (nn * nn);
     const int nb = n_bins();
-    timed("k_spec_sums", (double)F_ * nx_ * ny_ * nzh_ * sizeof(C), [&] {
-      hipLaunchKernelGGL(k_spec_sums<T>, dim3(nx_), dim3(STAT_THREADS), 0, s_, g_, ptrs(q_), dkx_,
-                         dky_, dkz_, S_, inn2, part);
-    });
     ShellArgs sa;
     sa.equal_box = (p_.lx == p_.ly && p_.ly == p_.lz) ? 1 : 0;
     const double lm = std::max(p_.lx, std::max(p_.ly, p_.lz));
     sa.fx = lm / p_.lx; sa.fy = lm / p_.ly; sa.fz = lm / p_.lz;
-    timed("k_spectrum", (double)F_ * nx_ * ny_ * nzh_ * sizeof(C), [&] {
-      hipLaunchKernelGGL(k_spectrum<T>, dim3(nx_), dim3(STAT_THREADS), 0, s_, g_, ptrs(q_), S_, nb, sa,
-                         inn2, spec);
+    // as many waves per plane as have room for their bins (one block per CU, at most 144 KiB of them);
+    // shells too many for four waves go to k_spectrum.  The waves fix the order of the sums, so they
+    // are the same with and without the spectrum.
+    const size_t wave_bins = sizeof(double) * (size_t)(1 + S_) * nb, room = 144 * 1024;
+    int threads = SPEC_THREADS;
+    while (threads > 256 && (threads / 64) * wave_bins > room) threads /= 2;
+    const bool fits = (threads / 64) * wave_bins <= room, bins = spec && fits;
+    if (!fits) threads = SPEC_THREADS;
+    timed("k_spec_sums", (double)F_ * nx_ * ny_ * nzh_ * sizeof(C), [&] {
+      if (bins)
+        hipLaunchKernelGGL((k_spectral_stats<T, true>), dim3(nx_), dim3(threads), (threads / 64) * wave_bins, s_, g_,
+                           ptrs(q_), dkx_, dky_, dkz_, S_, nb, sa, inn2, part, spec);
+      else
+        hipLaunchKernelGGL((k_spectral_stats<T, false>), dim3(nx_), dim3(threads), 0, s_, g_, ptrs(q_), dkx_,
+                           dky_, dkz_, S_, nb, sa, inn2, part, (double*)nullptr);
     });
+    if (spec && !bins)
+      timed("k_spectrum", (double)F_ * nx_ * ny_ * nzh_ * sizeof(C), [&] {
+        hipLaunchKernelGGL(k_spectrum<T>, dim3(nx_), dim3(STAT_THREADS), 0, s_, g_, ptrs(q_), S_, nb, sa,
+                           inn2, spec);
+      });
     for (int f = 0; f < F_; ++f) {
       GNSS_HIP(hipMemcpyAsync(ws_[0], q_[f], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
       inv3d(ws_[0], phys_[f], false);
     }
     RPtrs<T> pp{};
     for (int f = 0; f < F_; ++f) pp.p[f] = phys_[f];
-    timed("k_plane_stats", (double)F_ * nph_ * sizeof(T) * 2, [&] {
-      hipLaunchKernelGGL(k_plane_stats<T>, dim3(ny_), dim3(STAT_THREADS), 0, s_, g_, pp, S_,
+    timed("k_plane_stats", (double)F_ * nph_ * sizeof(T), [&] {
+      hipLaunchKernelGGL(k_plane_stats<T>, dim3(ny_), dim3(PLANE_THREADS), 0, s_, g_, pp, S_,
                          nx_ / p_.lx, ny_ / p_.ly, nz_ / p_.lz, prof, cmax);
     });
   }
@@ -1071,6 +1069,7 @@ class Engine : public EngineBase {
     dalloc(d_spec_, sizeof(double) * (size_t)nx_ * (1 + S_) * nb);
     dalloc(d_prof_, sizeof(double) * (size_t)(7 + 3 * S_) * ny_);
     dalloc(d_cmax_, sizeof(double) * 2 * ny_);
+    dalloc(d_fin_, sizeof(double) * (SPEC_NQ + 2 + (size_t)(1 + S_) * nb));
     dalloc(d_flag_, sizeof(int));
     // twiddle tables for every length the passes use
     for (int L : {nx_, ny_, nz_, nz_ / 2}) {
@@ -1936,7 +1935,7 @@ class Engine : public EngineBase {
   std::map<int, C*> tw_;
   double *dkx_ = nullptr, *dky_ = nullptr, *dkz_ = nullptr;
   T *tkx_ = nullptr, *tky_ = nullptr, *tkz_ = nullptr;
-  double *d_part_ = nullptr, *d_spec_ = nullptr, *d_prof_ = nullptr, *d_cmax_ = nullptr;
+  double *d_part_ = nullptr, *d_spec_ = nullptr, *d_prof_ = nullptr, *d_cmax_ = nullptr, *d_fin_ = nullptr;
   int* d_flag_ = nullptr;
   void* scratch_ = nullptr;
   size_t scratch_n_ = 0;

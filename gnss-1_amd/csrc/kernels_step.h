@@ -273,46 +273,6 @@ __device__ __forceinline__ void block_sum(const double (&acc)[NQ], double* sh, d
 
 constexpr int SPEC_NQ = 4 + 2 * 4;
 
-// Sums per kx plane (calcVrms/Epsilon/IntegralLength/ScalarDissipation kernels,
-// statistics.cu:1494-1845): [0] sum w|u|^2, [1] sum w k^2|u|^2, [2] sum w|u|^2/(2|k|),
-// [3] sum w|k.u|^2, [4+2s] sum w k^2|phi|^2, [5+2s] sum_{k!=0} w|phi|^2 — all divided by NN^2.
-template <typename T>
-__global__ void __launch_bounds__(STAT_THREADS)
-k_spec_sums(Geom g, CPtrs<T> q, const double* __restrict__ kxv, const double* __restrict__ kyv,
-            const double* __restrict__ kzv, int S, double inn2, double* __restrict__ part) {
-  __shared__ double sh[SPEC_NQ * STAT_THREADS];
-  const int ix = blockIdx.x;
-  double acc[SPEC_NQ];
-  for (int qq = 0; qq < SPEC_NQ; ++qq) acc[qq] = 0.0;
-  const double kx = kxv[ix];
-  const long long n = (long long)g.ny * g.nzh;
-  for (long long i = threadIdx.x; i < n; i += STAT_THREADS) {
-    const int iy = (int)(i / g.nzh), iz = (int)(i % g.nzh);
-    const long long o = ((long long)ix * g.ny + iy) * g.kzs + iz;
-    const double ky = kyv[iy], kz = kzv[iz];
-    const double k2 = kx * kx + ky * ky + kz * kz;
-    const double w = (iz == 0 || 2 * iz == g.nz) ? 1.0 : 2.0;
-    const cx<T> u = q.p[0][o], v = q.p[1][o], ww = q.p[2][o];
-    const double ux = u.x, uy = u.y, vx = v.x, vy = v.y, wx = ww.x, wy = ww.y;
-    const double e = (ux * ux + uy * uy + vx * vx + vy * vy + wx * wx + wy * wy) * inn2;
-    const double dr = kx * ux + ky * vx + kz * wx, di = kx * uy + ky * vy + kz * wy;
-    acc[0] += w * e;
-    acc[1] += w * k2 * e;
-    if (k2 > 0) acc[2] += w * e / (2.0 * sqrt(k2));
-    acc[3] += w * (dr * dr + di * di) * inn2;
-    for (int s = 0; s < S; ++s) {
-      const cx<T> ph = q.p[3 + s][o];
-      const double pr = ph.x, pi = ph.y;
-      const double ep = (pr * pr + pi * pi) * inn2;
-      acc[4 + 2 * s] += w * k2 * ep;
-      if (k2 > 0) acc[5 + 2 * s] += w * ep;
-    }
-  }
-  double tot[SPEC_NQ];
-  block_sum<SPEC_NQ>(acc, sh, tot);
-  if (threadIdx.x < SPEC_NQ) part[(long long)ix * SPEC_NQ + threadIdx.x] = tot[threadIdx.x];
-}
-
 struct ShellArgs {
   int equal_box;        // 1: shell = nint(|m|) in integers
   double fx, fy, fz;    // else shell = nint(sqrt((mx fx)^2 + (my fy)^2 + (mz fz)^2))
@@ -333,8 +293,135 @@ __device__ __forceinline__ int shell_of(const ShellArgs& a, int mx, int my, int 
   return (int)floor(sqrt(x * x + y * y + z * z) + 0.5);
 }
 
-// Shell spectrum of one kx plane (the reference declares it but never computes it,
-// statistics.cu:1847-1934).  Thread b owns shell b: for each ky it walks the kz interval of
+// Shell of the modes (mx, my, mz) with the integer rule's 4 |m|^2 in 32 bits (|m_i| <= 512, so
+// 4 |m|^2 < 2^22 is exact in FP32): the hardware root is at most one off and put right in integers.
+__device__ __forceinline__ int shell_small(int mx, int my, int mz) {
+  const int v = 4 * (mx * mx + my * my + mz * mz);
+  int r = (int)__fsqrt_rn((float)v);
+  r -= r * r > v ? 1 : 0;
+  r += (r + 1) * (r + 1) <= v ? 1 : 0;
+  return (r + 1) / 2;
+}
+
+// Sums of one kx plane over ky and kz (calcVrms/Epsilon/IntegralLength/ScalarDissipation kernels,
+// statistics.cu:1494-1845): [0] sum w|u|^2, [1] sum w k^2|u|^2, [2] sum w|u|^2/(2|k|),
+// [3] sum w|k.u|^2, [4+2s] sum w k^2|phi|^2, [5+2s] sum_{k!=0} w|phi|^2 — all divided by NN^2; and,
+// with BINS, the shell spectrum of the plane (the reference declares it but never computes it,
+// statistics.cu:1847-1934) in the same read of the state.
+// A wave takes whole ky rows, lane = kz.  Along a row the shell index does not decrease, so the modes
+// of one shell are neighbouring lanes: a segmented scan over the wave leaves each shell's sum in its
+// last lane, which adds it to the wave's own bins in LDS (no two lanes of a step share a shell); the
+// bins of the waves are summed in wave order.  Every sum so has a fixed order.  Steps in which every
+// mode is zero (those the 2/3 rule removed: 70 to 85 % of a dealiased state) are only read.
+// Bound by the one read of the state: 512^3, one scalar, FP32 0.56 ms (3.8 TB/s), FP64 0.78 ms (5.5 TB/s);
+// as two kernels (a thread per shell walking the rows for its modes, and a pass of its own for the
+// sums) 5.5 and 5.9 ms.
+constexpr int SPEC_THREADS = 1024;
+template <typename T, bool BINS>
+__global__ void __launch_bounds__(SPEC_THREADS)
+k_spectral_stats(Geom g, CPtrs<T> q, const double* __restrict__ kxv, const double* __restrict__ kyv,
+                 const double* __restrict__ kzv, int S, int nb, ShellArgs sa, double inn2,
+                 double* __restrict__ part, double* __restrict__ spec) {
+  extern __shared__ unsigned char smem_raw[];
+  double* bins = reinterpret_cast<double*>(smem_raw);  // [wave][1 + S][nb]
+  __shared__ double wsum[SPEC_THREADS / 64][SPEC_NQ];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int ix = blockIdx.x, mx = mode_of(ix, g.nx);
+  const int per = (1 + S) * nb;
+  double* mine = bins + (long long)wave * per;
+  if (BINS) {
+    for (int i = lane; i < per; i += 64) mine[i] = 0.0;
+    lds_sync<true>();
+  }
+  double acc[SPEC_NQ];
+#pragma unroll
+  for (int qq = 0; qq < SPEC_NQ; ++qq) acc[qq] = 0.0;
+  const double kx = kxv[ix];
+  const int nch = (g.nzh + 63) / 64;
+  for (int st = wave; st < g.ny * nch; st += nw) {
+    const int iy = st / nch, iz = (st % nch) * 64 + lane;
+    const bool on = iz < g.nzh;
+    const long long o = ((long long)ix * g.ny + iy) * g.kzs + (on ? iz : 0);
+    cx<T> f[MAXF];
+#pragma unroll
+    for (int i = 0; i < MAXF; ++i) f[i] = (on && i < 3 + S) ? ld_s(&q.p[i][o]) : mk<T>(0, 0);
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < MAXF; ++i) any = any || f[i].x != (T)0 || f[i].y != (T)0;
+    if (!__any(any)) continue;
+    const double ky = kyv[iy], kz = on ? kzv[iz] : 0.0;
+    const double k2 = kx * kx + ky * ky + kz * kz;
+    const double w = (iz == 0 || 2 * iz == g.nz) ? 1.0 : 2.0;
+    double e[1 + 4];
+    {
+      const double ux = f[0].x, uy = f[0].y, vx = f[1].x, vy = f[1].y, wx = f[2].x, wy = f[2].y;
+      e[0] = (ux * ux + uy * uy + vx * vx + vy * vy + wx * wx + wy * wy) * inn2;
+      const double dr = kx * ux + ky * vx + kz * wx, di = kx * uy + ky * vy + kz * wy;
+      acc[0] += w * e[0];
+      acc[1] += w * k2 * e[0];
+      if (k2 > 0) acc[2] += w * e[0] / (2.0 * sqrt(k2));
+      acc[3] += w * (dr * dr + di * di) * inn2;
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const double pr = f[3 + s].x, pi = f[3 + s].y;
+      e[1 + s] = (pr * pr + pi * pi) * inn2;
+      if (s < S) {
+        acc[4 + 2 * s] += w * k2 * e[1 + s];
+        if (k2 > 0) acc[5 + 2 * s] += w * e[1 + s];
+      }
+    }
+    if constexpr (BINS) {
+      const int my = mode_of(iy, g.ny), mz = iz < (g.nz >> 1) ? iz : -(g.nz >> 1);
+      const int sh = !on ? 0x7FFFFFFF : (sa.equal_box ? shell_small(mx, my, mz) : shell_of(sa, mx, my, mz));
+#pragma unroll
+      for (int s = 0; s < 5; ++s) e[s] *= 0.5 * w;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const bool same = __shfl_up(sh, d) == sh && lane >= d;
+        if (!__any(same)) break;
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+          if (s > S) break;
+          const double up = __shfl_up(e[s], d);
+          if (same) e[s] += up;
+        }
+      }
+      const int next = __shfl_down(sh, 1);
+      if (on && (lane == 63 || next != sh)) {
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+          if (s > S) break;
+          mine[s * nb + sh] += e[s];
+        }
+      }
+      lds_sync<true>();
+    }
+  }
+#pragma unroll
+  for (int qq = 0; qq < SPEC_NQ; ++qq) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) acc[qq] += __shfl_down(acc[qq], d);
+    if (lane == 0) wsum[wave][qq] = acc[qq];
+  }
+  __syncthreads();
+  if (threadIdx.x < SPEC_NQ) {
+    double t = 0.0;
+    for (int i = 0; i < nw; ++i) t += wsum[i][threadIdx.x];
+    part[(long long)ix * SPEC_NQ + threadIdx.x] = t;
+  }
+  if constexpr (BINS) {
+    for (int j = threadIdx.x; j < per; j += blockDim.x) {
+      double t = 0.0;
+      for (int i = 0; i < nw; ++i) t += bins[(long long)i * per + j];
+      spec[(long long)ix * per + j] = t;
+    }
+  }
+}
+
+// The spectrum where a plane's bins do not fit the LDS (boxes with very unequal sides, whose shell
+// count grows with the longest over the shortest): shells of one kx plane.
+// Thread b owns shell b: for each ky it walks the kz interval of
 // that shell (the shell index is non-decreasing in kz), so every sum has a fixed order.
 template <typename T>
 __global__ void __launch_bounds__(STAT_THREADS)
@@ -372,79 +459,134 @@ k_spectrum(Geom g, CPtrs<T> q, int S, int nb, ShellArgs sa, double inn2, double*
   }
 }
 
-// x-z plane averages at one y (calcYprof_kernel_2D, statistics.cu:1936-1977), two passes:
-// means, then <u'u'>, <v'v'>, <w'w'>, <u'v'>, <phi'phi'>, <v'phi'>, plus the CFL and |u| maxima.
+// x-z plane averages at one y (calcYprof_kernel_2D, statistics.cu:1936-1977): means, <u'u'>, <v'v'>,
+// <w'w'>, <u'v'>, <phi'phi'>, <v'phi'>, plus the CFL and |u| maxima, in one read of the plane: sums
+// of d = f - c and of their products, with c the mean of eight sample rows, so that |mean - c| lies
+// within the fluctuations and <f'g'> = <d_f d_g> - <d_f><d_g> cancels nothing (all in FP64, fixed
+// order).  16-byte loads (nz is a multiple of 8).  Bound by that read: 512^3, one scalar, FP32 0.38 ms
+// (5.6 TB/s), FP64 0.79 ms; as two passes of scalar loads 3.1 and 3.3 ms.
+constexpr int PLANE_THREADS = 1024;
+constexpr int PLANE_NQ = MAXF + 4 + 2 * 4;
 template <typename T>
-__global__ void __launch_bounds__(STAT_THREADS)
+__global__ void __launch_bounds__(PLANE_THREADS)
 k_plane_stats(Geom g, RPtrs<T> ph, int S, double idx_, double idy_, double idz_,
               double* __restrict__ prof, double* __restrict__ cmax) {
-  constexpr int NQ = 4 + 2 * 4;
-  __shared__ double sh[NQ * STAT_THREADS];
-  __shared__ double mean[3 + 4];
-  const int y = blockIdx.x;
-  const int F = 3 + S;
-  const long long n = (long long)g.nx * g.nz;
-  const double inv = 1.0 / (double)n;
-  double acc[NQ];
-  for (int qq = 0; qq < NQ; ++qq) acc[qq] = 0.0;
-  for (long long i = threadIdx.x; i < n; i += STAT_THREADS) {
-    const int x = (int)(i / g.nz), z = (int)(i % g.nz);
-    const long long o = ((long long)x * g.ny + y) * g.nz + z;
-    for (int f = 0; f < F; ++f) acc[f] += (double)ph.p[f][o];
+  constexpr int V = 16 / (int)sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(V)));
+  __shared__ double wsum[PLANE_THREADS / 64][PLANE_NQ + 2];
+  __shared__ double tot[PLANE_NQ + 2];
+  const int y = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nv = g.nz / V, nt = blockDim.x;
+  auto load = [&](int i, vec* f) {
+    const int x = i / nv, z = i - x * nv;
+    const long long o = ((long long)x * g.ny + y) * nv + z;
+#pragma unroll
+    for (int k = 0; k < MAXF; ++k)
+      if (k < 3 + S) f[k] = reinterpret_cast<const vec*>(ph.p[k])[o];
+  };
+  // totals of the first n entries of acc over the block (every thread reads them in tot)
+  auto reduce = [&](double* acc, int q) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) acc[0] += __shfl_down(acc[0], d);
+    if (lane == 0) wsum[wave][q] = acc[0];
+  };
+  const int rows = g.nx < 8 ? g.nx : 8, xs = g.nx / rows;
+  double c[MAXF];
+#pragma unroll
+  for (int k = 0; k < MAXF; ++k) c[k] = 0.0;
+  for (int i = tid; i < rows * nv; i += nt) {
+    vec f[MAXF];
+    const int r = i / nv;
+    load(r * xs * nv + (i - r * nv), f);
+#pragma unroll
+    for (int k = 0; k < MAXF; ++k)
+      if (k < 3 + S)
+#pragma unroll
+        for (int j = 0; j < V; ++j) c[k] += (double)f[k][j];
   }
-  double tot[NQ];
-  block_sum<NQ>(acc, sh, tot);
-  if (threadIdx.x < F) mean[threadIdx.x] = tot[threadIdx.x] * inv;
+#pragma unroll
+  for (int k = 0; k < MAXF; ++k) reduce(&c[k], k);
   __syncthreads();
-  for (int qq = 0; qq < NQ; ++qq) acc[qq] = 0.0;
+  if (tid < MAXF) {
+    double t = 0.0;
+    for (int i = 0; i < nt / 64; ++i) t += wsum[i][tid];
+    tot[tid] = t / ((double)rows * g.nz);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < MAXF; ++k) c[k] = tot[k];
+  double acc[PLANE_NQ];
+#pragma unroll
+  for (int k = 0; k < PLANE_NQ; ++k) acc[k] = 0.0;
   double cm = 0.0, um = 0.0;
-  for (long long i = threadIdx.x; i < n; i += STAT_THREADS) {
-    const int x = (int)(i / g.nz), z = (int)(i % g.nz);
-    const long long o = ((long long)x * g.ny + y) * g.nz + z;
-    const double u = ph.p[0][o], v = ph.p[1][o], w = ph.p[2][o];
-    const double du = u - mean[0], dv = v - mean[1], dw = w - mean[2];
-    acc[0] += du * du;
-    acc[1] += dv * dv;
-    acc[2] += dw * dw;
-    acc[3] += du * dv;
-    for (int s = 0; s < S; ++s) {
-      const double dp = (double)ph.p[3 + s][o] - mean[3 + s];
-      acc[4 + 2 * s] += dp * dp;
-      acc[5 + 2 * s] += dv * dp;
+  const int n = g.nx * nv;
+  for (int i = tid; i < n; i += nt) {
+    vec f[MAXF];
+    load(i, f);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const double u = f[0][j], v = f[1][j], w = f[2][j];
+      const double du = u - c[0], dv = v - c[1], dw = w - c[2];
+      acc[0] += du;
+      acc[1] += dv;
+      acc[2] += dw;
+      acc[MAXF] += du * du;
+      acc[MAXF + 1] += dv * dv;
+      acc[MAXF + 2] += dw * dw;
+      acc[MAXF + 3] += du * dv;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s < S) {
+          const double dp = (double)f[3 + s][j] - c[3 + s];
+          acc[3 + s] += dp;
+          acc[MAXF + 4 + 2 * s] += dp * dp;
+          acc[MAXF + 5 + 2 * s] += dv * dp;
+        }
+      cm = fmax(cm, fabs(u) * idx_ + fabs(v) * idy_ + fabs(w) * idz_);
+      um = fmax(um, fmax(fabs(u), fmax(fabs(v), fabs(w))));
     }
-    const double cf = fabs(u) * idx_ + fabs(v) * idy_ + fabs(w) * idz_;
-    cm = fmax(cm, cf);
-    um = fmax(um, fmax(fabs(u), fmax(fabs(v), fabs(w))));
   }
-  block_sum<NQ>(acc, sh, tot);
-  // max reductions (order independent)
-  __syncthreads();
-  sh[threadIdx.x] = cm;
-  sh[STAT_THREADS + threadIdx.x] = um;
-  __syncthreads();
-  for (int s = STAT_THREADS / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-      sh[STAT_THREADS + threadIdx.x] = fmax(sh[STAT_THREADS + threadIdx.x], sh[STAT_THREADS + threadIdx.x + s]);
-    }
-    __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PLANE_NQ; ++k) reduce(&acc[k], k);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    cm = fmax(cm, __shfl_down(cm, d));
+    um = fmax(um, __shfl_down(um, d));
   }
-  if (threadIdx.x == 0) {
+  if (lane == 0) {
+    wsum[wave][PLANE_NQ] = cm;
+    wsum[wave][PLANE_NQ + 1] = um;
+  }
+  __syncthreads();
+  const double inv = 1.0 / ((double)g.nx * g.nz);
+  if (tid < PLANE_NQ) {
+    double t = 0.0;
+    for (int i = 0; i < nt / 64; ++i) t += wsum[i][tid];
+    tot[tid] = t * inv;
+  } else if (tid < PLANE_NQ + 2) {
+    double t = 0.0;
+    for (int i = 0; i < nt / 64; ++i) t = fmax(t, wsum[i][tid]);
+    tot[tid] = t;
+  }
+  __syncthreads();
+  if (tid == 0) {
     const int ny = g.ny;
-    prof[0 * ny + y] = mean[0];
-    prof[1 * ny + y] = mean[1];
-    prof[2 * ny + y] = mean[2];
-    prof[3 * ny + y] = tot[0] * inv;
-    prof[4 * ny + y] = tot[1] * inv;
-    prof[5 * ny + y] = tot[2] * inv;
-    prof[6 * ny + y] = tot[3] * inv;
+    const double* m = tot;          // <d_f>
+    const double* p = tot + MAXF;   // <d_f d_g>
+    prof[0 * ny + y] = c[0] + m[0];
+    prof[1 * ny + y] = c[1] + m[1];
+    prof[2 * ny + y] = c[2] + m[2];
+    prof[3 * ny + y] = p[0] - m[0] * m[0];
+    prof[4 * ny + y] = p[1] - m[1] * m[1];
+    prof[5 * ny + y] = p[2] - m[2] * m[2];
+    prof[6 * ny + y] = p[3] - m[0] * m[1];
     for (int s = 0; s < S; ++s) {
-      prof[(7 + 3 * s) * ny + y] = mean[3 + s];
-      prof[(8 + 3 * s) * ny + y] = tot[4 + 2 * s] * inv;
-      prof[(9 + 3 * s) * ny + y] = tot[5 + 2 * s] * inv;
+      prof[(7 + 3 * s) * ny + y] = tot[3 + s] + (s == 0 ? c[3] : s == 1 ? c[4] : s == 2 ? c[5] : c[6]);
+      prof[(8 + 3 * s) * ny + y] = p[4 + 2 * s] - m[3 + s] * m[3 + s];
+      prof[(9 + 3 * s) * ny + y] = p[5 + 2 * s] - m[1] * m[3 + s];
     }
-    cmax[2 * y] = sh[0];
-    cmax[2 * y + 1] = sh[STAT_THREADS];
+    cmax[2 * y] = tot[PLANE_NQ];
+    cmax[2 * y + 1] = tot[PLANE_NQ + 1];
   }
 }
 
@@ -997,28 +1139,28 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
   }
 }
 
-// The reductions of the allocation-free statistics call, on the device and in the order the host
-// sums the same partials for gnss_stats (so both give the same bits): fin[q] = sum over x of
-// part[x][q] (q < SPEC_NQ); fin[SPEC_NQ], fin[SPEC_NQ + 1] = max over y of the CFL sum and of
-// max |u_i|; fin[SPEC_NQ + 2 + j] = sum over x of spec[x][j] (j < nspec shell entries).
-static __global__ void __launch_bounds__(STAT_THREADS)
+// Sums of the per-plane partials in plane order, a thread per result: fin[q] = sum over x of
+// part[x][q] (q < SPEC_NQ); fin[SPEC_NQ], fin[SPEC_NQ + 1] = max over y of the CFL sum and of max |u_i|;
+// fin[SPEC_NQ + 2 + j] = sum over x of spec[x][j] (j < nspec shell entries).  Eight loads go out
+// ahead of their additions (a serial chain of loads cost 1 us each).
+static __global__ void __launch_bounds__(64)
 k_stats_reduce(const double* __restrict__ part, const double* __restrict__ spec, const double* __restrict__ cmax,
                int nx, int ny, int nspec, double* __restrict__ fin) {
-  const int t = threadIdx.x;
-  if (t < SPEC_NQ) {
-    double acc = 0.0;
-    for (int x = 0; x < nx; ++x) acc += part[(long long)x * SPEC_NQ + t];
-    fin[t] = acc;
-  } else if (t < SPEC_NQ + 2) {
-    double m = 0.0;
-    for (int y = 0; y < ny; ++y) m = fmax(m, cmax[2 * y + (t - SPEC_NQ)]);
-    fin[t] = m;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= SPEC_NQ + 2 + nspec) return;
+  const bool mx = t == SPEC_NQ || t == SPEC_NQ + 1;
+  const double* src = t < SPEC_NQ ? part + t : (mx ? cmax + (t - SPEC_NQ) : spec + (t - SPEC_NQ - 2));
+  const long long stride = t < SPEC_NQ ? SPEC_NQ : (mx ? 2 : nspec);
+  const int n = mx ? ny : nx;  // multiples of 8
+  double acc = 0.0;
+  for (int i = 0; i < n; i += 8) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = src[(i + k) * stride];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc = mx ? fmax(acc, v[k]) : acc + v[k];
   }
-  for (int j = t; j < nspec; j += STAT_THREADS) {
-    double acc = 0.0;
-    for (int x = 0; x < nx; ++x) acc += spec[(long long)x * nspec + j];
-    fin[SPEC_NQ + 2 + j] = acc;
-  }
+  fin[t] = acc;
 }
 
 // Plain copy (bandwidth reference): block b copies the contiguous chunk [b chunk, (b + 1) chunk)
