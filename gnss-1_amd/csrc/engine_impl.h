@@ -71,6 +71,18 @@ class Engine : public EngineBase {
     mask_factors(nx_, ny_, nz_, ax, ay, az, g2);
     g_.ax = ax; g_.ay = ay; g_.az = az; g_.g2 = g2;
     kz_lim_ = std::min(round_up(g_.keep_z + 1, cmax), kzs_);
+    sph_.shift = sizeof(T) == 8 ? 3 : 4;  // cmax
+    sph_.r2 = (float)((double)g_.g2 / 9.0);
+    sph_.ay = (float)g_.ay;
+    sph_.az = (float)g_.az;
+    sph_.rax = (float)(1.0 / (double)g_.ax);
+    static_assert(SPHERE_BLOCKS >= 344 / 8, "a block bound for every kz tile of the longest row");
+    for (int b = 0; b < kz_lim_ / cmax; ++b) {
+      int m = -1;
+      const long long z = (long long)b * cmax * g_.az;
+      while (m < g_.keep_y && 9 * ((m + 1) * g_.ay * (m + 1) * g_.ay + z * z) <= g_.g2) ++m;
+      sph_.ky[b] = (short)m;
+    }
     nsp_ = (long long)nx_ * ny_ * kzs_;
     nph_ = (long long)nx_ * ny_ * nz_;
     GNSS_HIP(hipStreamCreateWithFlags(&s_, hipStreamNonBlocking));
@@ -1139,6 +1151,7 @@ class Engine : public EngineBase {
     int nchunks;     // column chunks processed
     int outer_keep;  // kept-mode outer map (x pass: over ky), -1 = all
     int in_keep, out_keep;
+    bool pruned() const { return in_keep >= 0 || out_keep >= 0; }
   };
 
   // the pass over nf fields: persistent blocks over all their tiles (cp), else one launch per field
@@ -1261,6 +1274,7 @@ class Engine : public EngineBase {
     a.nchunks = sp.nchunks;
     a.in_keep = sp.in_keep;
     a.out_keep = sp.out_keep;
+    if (sp.pruned()) a.sph = sphere(sp.axis);
     batch_outer(a);
     int G = std::max(1, 256 / (CC * TPC));
     while (G > 1 && (long long)G * L * CC * (long long)sizeof(C) > LDS_MAX) --G;
@@ -1556,6 +1570,7 @@ class Engine : public EngineBase {
     ax.in_keep = g_.keep_x;
     ax.out_keep = -1;
     ax.G = 1;
+    ax.sph = sphere(0);
     ColArgs ay;
     ay.estride = kzs_;
     ay.ostride = (long long)ny_ * kzs_;
@@ -1566,12 +1581,20 @@ class Engine : public EngineBase {
     ay.in_keep = g_.keep_y;
     ay.out_keep = -1;
     ay.G = 1;
+    ay.sph = sphere(1);
     batch_outer(ax);
     batch_outer(ay);
     pair_pass(lx, nxe, ax, nx_, tkx_, "fft_x_inv_late", CC);
     pair_pass(ly, nye, ay, ny_, tky_, "fft_y_inv_late", CY);
   }
   int pair_chunk() const { return xc_; }
+  // The 2/3 rule's ellipsoid for a pruned pass over kx (axis 0) or ky (1) rows.  Off for the MFMA
+  // passes, which read and write whole boxes.
+  Sphere sphere(int axis) const {
+    Sphere s = sph_;
+    s.axis = (p_.flags & GNSS_FLAG_MFMA_R16) ? -1 : axis;
+    return s;
+  }
   // A pass of a batched step covers the outer indices of every member.
   void batch_outer(ColArgs& a) const {
     if (bm_ <= 1) return;
@@ -1579,109 +1602,46 @@ class Engine : public EngineBase {
     a.nouter *= bm_;
     a.mstride = nsp_;
   }
-  // With lp = 1 an entry's two outputs go through one launch (lp = 2: transformed one after the
-  // other through one LDS region, which halves the kernel's LDS; lp = 3: together, with the next
-  // tile's input loaded before they transform); with lp = 0 they are split into
-  // single-output entries that read the inputs again, the second outputs first (they read fields
-  // the first outputs overwrite in place).  Then one launch per (inputs, outputs) kind with cb,
-  // else one per entry.
-  void pair_pass(const PairList<T>& li, int n, ColArgs a, int L, const T* kv, const char* name, int CC) {
-    if (lp_) return pair_kinds(li, n, a, L, kv, name, CC);
-    PairList<T> first{}, second{};
-    int n1 = 0, n2 = 0;
-    for (int i = 0; i < n; ++i) {
-      const PairOp& op = li.op[i];
-      const bool first_uses_b = op.c[0] != 0 || op.d[0] != 0;
-      const PairOp o0{first_uses_b ? 2 : 1, 1, {op.a[0], 0}, {op.b[0], 0}, {op.c[0], 0}, {op.d[0], 0}};
-      first.A[n1] = li.A[i];
-      first.B[n1] = li.B[i];
-      first.out[0][n1] = first.out[1][n1] = li.out[0][i];
-      first.op[n1++] = o0;
-      if (op.nout == 2) {
-        const bool uses_b = op.c[1] != 0 || op.d[1] != 0;
-        PairOp o1{uses_b ? 2 : 1, 1, {op.a[1], 0}, {op.b[1], 0}, {op.c[1], 0}, {op.d[1], 0}};
-        second.A[n2] = li.A[i];
-        second.B[n2] = li.B[i];
-        second.out[0][n2] = second.out[1][n2] = li.out[1][i];
-        second.op[n2++] = o1;
-      }
-    }
-    pair_kinds(second, n2, a, L, kv, name, CC);
-    pair_kinds(first, n1, a, L, kv, name, CC);
-  }
-  void pair_kinds(const PairList<T>& li, int n, ColArgs a, int L, const T* kv, const char* name, int CC) {
+  void pair_pass(const PairList<T>& li, int n, const ColArgs& a, int L, const T* kv, const char* name, int CC) {
     auto rows = [&](int keep) { return keep < 0 ? L : std::min(L, 2 * keep + 1); };
     const double col = (double)a.nouter * a.nchunks * CC * sizeof(C);
-    static const int KIN[4] = {1, 1, 2, 2}, KOUT[4] = {1, 2, 2, 1};
-    for (int kind = 0; kind < 4; ++kind) {
-      const int nin = KIN[kind], nout = KOUT[kind];
-      std::vector<int> ents;
-      for (int i = 0; i < n; ++i)
-        if (li.op[i].nin == nin && li.op[i].nout == nout) ents.push_back(i);
-      const int groups = cb_ ? (ents.empty() ? 0 : 1) : (int)ents.size();
-      for (int gi = 0; gi < groups; ++gi) {
-        const int i0 = cb_ ? 0 : gi, i1 = cb_ ? (int)ents.size() : gi + 1;
-        PairList<T> sub{};
-        for (int i = i0; i < i1; ++i) {
-          const int j = ents[i], k = i - i0;
-          sub.A[k] = li.A[j];
-          sub.B[k] = li.B[j];
-          sub.out[0][k] = li.out[0][j];
-          sub.out[1][k] = li.out[1][j];
-          sub.op[k] = li.op[j];
-        }
-        const int m = i1 - i0;
-        timed(name, col * m * (nin * rows(a.in_keep) + nout * rows(a.out_keep)), [&] {
-          switch (L) {
-            case 16: pair_c<16>(sub, m, a, kv, CC, kind); break;
-            case 24: pair_c<24>(sub, m, a, kv, CC, kind); break;
-            case 32: pair_c<32>(sub, m, a, kv, CC, kind); break;
-            case 48: pair_c<48>(sub, m, a, kv, CC, kind); break;
-            case 64: pair_c<64>(sub, m, a, kv, CC, kind); break;
-            case 96: pair_c<96>(sub, m, a, kv, CC, kind); break;
-            case 128: pair_c<128>(sub, m, a, kv, CC, kind); break;
-            case 192: pair_c<192>(sub, m, a, kv, CC, kind); break;
-            case 256: pair_c<256>(sub, m, a, kv, CC, kind); break;
-            case 384: pair_c<384>(sub, m, a, kv, CC, kind); break;
-            case 512: pair_c<512>(sub, m, a, kv, CC, kind); break;
-            case 1024: pair_c<1024>(sub, m, a, kv, CC, kind); break;
-            default: throw Error(GNSS_ERR_UNSUPPORTED, "late pass length " + std::to_string(L));
-          }
-        });
+    double bytes = 0;
+    for (int i = 0; i < n; ++i) bytes += col * (li.op[i].nin * rows(a.in_keep) + li.op[i].nout * rows(a.out_keep));
+    timed(name, bytes, [&] {
+      switch (L) {
+        case 16: pair_c<16>(li, n, a, kv, CC); break;
+        case 24: pair_c<24>(li, n, a, kv, CC); break;
+        case 32: pair_c<32>(li, n, a, kv, CC); break;
+        case 48: pair_c<48>(li, n, a, kv, CC); break;
+        case 64: pair_c<64>(li, n, a, kv, CC); break;
+        case 96: pair_c<96>(li, n, a, kv, CC); break;
+        case 128: pair_c<128>(li, n, a, kv, CC); break;
+        case 192: pair_c<192>(li, n, a, kv, CC); break;
+        case 256: pair_c<256>(li, n, a, kv, CC); break;
+        case 384: pair_c<384>(li, n, a, kv, CC); break;
+        case 512: pair_c<512>(li, n, a, kv, CC); break;
+        case 1024: pair_c<1024>(li, n, a, kv, CC); break;
+        default: throw Error(GNSS_ERR_UNSUPPORTED, "late pass length " + std::to_string(L));
       }
-    }
+    });
   }
   template <int L>
-  void pair_c(const PairList<T>& li, int n, const ColArgs& a, const T* kv, int CC, int kind) {
+  void pair_c(const PairList<T>& li, int n, const ColArgs& a, const T* kv, int CC) {
     if constexpr (sizeof(T) == 8) {
-      if (CC == 8) pair_k<L, 8>(li, n, a, kv, kind);
-      else pair_k<L, 4>(li, n, a, kv, kind);
+      if (CC == 8) pair_launch<L, 8>(li, n, a, kv);
+      else pair_launch<L, 4>(li, n, a, kv);
     } else {
-      if (CC == 16) pair_k<L, 16>(li, n, a, kv, kind);
-      else pair_k<L, 8>(li, n, a, kv, kind);
+      if (CC == 16) pair_launch<L, 16>(li, n, a, kv);
+      else pair_launch<L, 8>(li, n, a, kv);
     }
   }
-  // two-output form of lp = 1, 2, 3
-  template <int L, int CC, int NIN>
-  void pair_k2(const PairList<T>& li, int n, const ColArgs& a, const T* kv) {
-    if (lp_ == 2) pair_launch<L, CC, NIN, 2, PAIR_SEQ>(li, n, a, kv);
-    else if (lp_ == 3) pair_launch<L, CC, NIN, 2, PAIR_BATCHED_PF>(li, n, a, kv);
-    else pair_launch<L, CC, NIN, 2, PAIR_BATCHED>(li, n, a, kv);
-  }
   template <int L, int CC>
-  void pair_k(const PairList<T>& li, int n, const ColArgs& a, const T* kv, int kind) {
-    if (kind == 0) pair_launch<L, CC, 1, 1, PAIR_BATCHED>(li, n, a, kv);
-    else if (kind == 1) pair_k2<L, CC, 1>(li, n, a, kv);
-    else if (kind == 2) pair_k2<L, CC, 2>(li, n, a, kv);
-    else pair_launch<L, CC, 2, 1, PAIR_BATCHED>(li, n, a, kv);
-  }
-  template <int L, int CC, int NIN, int NOUT, int FORM>
   void pair_launch(const PairList<T>& li, int n, ColArgs a, const T* kv) {
     constexpr int TPC = L / Plan<L>::E;
-    // two batched outputs use two LDS regions, and the twiddles have a copy after them: up to the
-    // 160 KiB a gfx950 workgroup can hold
+    // one data region per group, and the twiddles' copy after them: up to the 160 KiB a gfx950
+    // workgroup can hold
     constexpr long long PAIR_LDS_MAX = 160 * 1024;
-    const long long region = (long long)(NOUT == 2 && FORM == PAIR_SEQ ? 1 : NOUT) * L * CC * (long long)sizeof(C);
+    const long long region = (long long)L * CC * (long long)sizeof(C);
     const long long twb = (long long)L * (long long)sizeof(C);
     int G = std::max(1, 256 / (CC * TPC));
     while (G > 1 && G * region + twb > PAIR_LDS_MAX) --G;
@@ -1694,8 +1654,8 @@ class Engine : public EngineBase {
     const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
     const long long per_cu = std::max<long long>(1, std::min<long long>(160 * 1024 / (long long)lds, 2048 / threads));
     const long long grid = std::min<long long>(blocks * n, per_cu * n_cu_);
-    hipLaunchKernelGGL((k_inv_pair_pipe<T, L, CC, NIN, NOUT, FORM>), dim3((unsigned)grid), dim3(threads), lds, s_, li,
-                       kv, tw_.at(L), a, (int)blocks, (int)(blocks * n));
+    hipLaunchKernelGGL((k_inv_late<T, L, CC>), dim3((unsigned)grid), dim3(threads), lds, s_, li, kv, tw_.at(L), a,
+                       (int)blocks, (int)(blocks * n));
   }
 
   // x inverse passes of all work fields formed from the state (modes 2 and 3): one-input and
@@ -1727,6 +1687,7 @@ class Engine : public EngineBase {
     a.nchunks = kz_lim_ / xc_;
     a.in_keep = g_.keep_x;
     a.out_keep = -1;
+    a.sph = sphere(0);
     a.G = 1;
     const int nin = two ? 2 : 1;
     const double bytes = n * (double)a.nouter * a.nchunks * xc_ * (nin * (2.0 * g_.keep_x + 1) + nx_) * sizeof(C);
@@ -1767,7 +1728,7 @@ class Engine : public EngineBase {
                          g_, ptrs(q_), ptrs(ws_), tkx_, tky_, tkz_, tw_.at(L), scalar, nchunks, G);
     else
       hipLaunchKernelGGL((k_xfwd_rk<T, L, CC, GRP == 0>), dim3((unsigned)blocks), dim3(CC * TPC * G), lds, s_, g_,
-                         ptrs(q_), ptrs(dq_), ptrs(nl_), tkx_, tky_, tkz_, tw_.at(L), rc, scalar, nchunks, G);
+                         ptrs(q_), ptrs(dq_), ptrs(nl_), tkx_, tky_, tkz_, tw_.at(L), rc, sphere(0), scalar, nchunks, G);
   }
   template <int L, int CC>
   void xgrp_k(bool pro, int G, int nchunks, int grp, const RkCoef& rc) {
@@ -1929,6 +1890,7 @@ class Engine : public EngineBase {
   int kz_lim_ = 0;
   long long nsp_ = 0, nph_ = 0;
   Geom g_{};
+  Sphere sph_{};
   hipStream_t s_ = nullptr;
   std::vector<C*> q_, dq_, ws_, nl_;
   std::vector<T*> wp_, nlp_, phys_;

@@ -46,6 +46,20 @@ __device__ __forceinline__ bool row_kept(int p, int n, int keep) {
   return (m < 0 ? -m : m) <= keep;
 }
 
+// The 2/3 rule keeps an ellipsoid of modes, whose largest ky falls with kz: 21 % of the (ky, kz) columns
+// of the kept box hold removed modes only, and half of its modes are outside.  The x passes of a
+// substage leave those columns alone, the y passes take their rows for zeros (inverse) or do not
+// store them (forward), and the x passes read and write the rows inside only.  ky[b]: the largest kept
+// |ky| of the kz block b of 2^shift entries (the widest column tile), the same for every pass, so that
+// a pass never reads a column its predecessor left out.
+constexpr int SPHERE_BLOCKS = 64;
+struct Sphere {
+  int axis = -1;               // pass over rows of kx (0) or ky (1); -1: no ellipsoid
+  int shift = 0;
+  float r2 = 0, ay = 0, az = 0, rax = 0;  // ellipsoid radius^2 and mode scales: (mx/rax)^2 + (my ay)^2 + (mz az)^2 <= r2
+  short ky[SPHERE_BLOCKS] = {};
+};
+
 struct ColArgs {
   long long estride;   // distance between consecutive elements along the transformed axis
   long long ostride;   // distance between consecutive outer indices
@@ -58,7 +72,33 @@ struct ColArgs {
   int out_keep;        // -1 all rows, else only rows with |mode| <= out_keep are stored
   int nouter_m = 0;    // batched contexts: outer indices per member (0: one member)
   long long mstride = 0;  // batched contexts: elements between members
+  Sphere sph{};        // bounds of the 2/3 rule's ellipsoid, for pruned passes (axis < 0: none)
 };
+
+// What one tile of a strided pass has to do under the ellipsoid: nothing (dead: an x pass's column of
+// modes that are all removed), or the rows with |mode| <= keep only.  om: the tile's outer index (storage
+// order), chunk0: its first column.
+struct TileRows {
+  bool live;
+  int keep;  // -1: all rows
+};
+__device__ __forceinline__ TileRows tile_rows(const Sphere& s, int outer, int outer_n, int chunk0, int box_keep) {
+  TileRows r{true, box_keep};
+  if (s.axis < 0) return r;
+  const int k = s.ky[chunk0 >> s.shift];
+  if (s.axis == 1) {
+    r.keep = box_keep < 0 ? -1 : k;
+  } else {
+    const int my = mode_of(outer, outer_n);
+    r.live = (my < 0 ? -my : my) <= k;
+    const float y = (float)my * s.ay, z = (float)((chunk0 >> s.shift) << s.shift) * s.az;
+    // one row more than the root says: its rounding may not take a kept row away, and the rows
+    // outside the ellipsoid hold zeros
+    const int b = (int)(sqrtf(fmaxf(s.r2 - y * y - z * z, 0.0f)) * s.rax) + 1;
+    r.keep = b < box_keep ? b : box_keep;
+  }
+  return r;
+}
 
 // C2C pass along a strided axis of length L, in place.  Block = G x TPC x C threads.
 // Largest block a pass launches: one transform group, or 256 threads of several groups.
@@ -77,24 +117,28 @@ k_col(cx<T>* __restrict__ data, const cx<T>* __restrict__ tw, ColArgs a) {
   const int g = tid / (C * TPC);
   const int chunk = blockIdx.x % a.nchunks;
   const int o = (blockIdx.x / a.nchunks) * a.G + g;
-  const bool active = o < a.nouter;
+  bool active = o < a.nouter;
   int om = active ? o : 0;
   const long long mo = member_split(om, a.nouter_m, a.mstride);
-  const long long io = outer_index(om, a.outer_keep, a.outer_n);
-  cx<T>* base = data + mo + io * a.ostride + (long long)chunk * C + c;
+  const int io = outer_index(om, a.outer_keep, a.outer_n);
+  const TileRows in = tile_rows(a.sph, io, a.outer_n, chunk * C, a.in_keep);
+  active = active && in.live;
+  if (a.G == 1 && !active) return;
+  cx<T>* base = data + mo + (long long)io * a.ostride + (long long)chunk * C + c;
   cx<T> v[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = t + e * TPC;
-    if (active && row_kept(p, L, a.in_keep)) v[e] = ld_s(&base[(long long)p * a.estride]);
+    if (active && row_kept(p, L, in.keep)) v[e] = ld_s(&base[(long long)p * a.estride]);
     else v[e] = mk<T>(0, 0);
   }
   fft<T, L, SIGN>(v, lds, t, LdsCol{g * L * C + c, C}, tw);
   if (!active) return;
+  const int out_keep = tile_rows(a.sph, io, a.outer_n, chunk * C, a.out_keep).keep;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = t + e * TPC;
-    if (row_kept(p, L, a.out_keep)) st_s(&base[(long long)p * a.estride], v[e]);
+    if (row_kept(p, L, out_keep)) st_s(&base[(long long)p * a.estride], v[e]);
   }
 }
 
@@ -118,26 +162,40 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   const int c = tid % C;
   const int t = (tid / C) % TPC;
   const int g = tid / (C * TPC);
-  auto base_of = [&](int tile, bool& active) {
+  auto base_of = [&](int tile, TileRows& r, int box_keep) {
     const int f = tile / tpf, lt = tile % tpf;
     const int chunk = lt % a.nchunks;
     const int o = (lt / a.nchunks) * a.G + g;
-    active = o < a.nouter;
+    const bool active = o < a.nouter;
     int om = active ? o : 0;
     const long long mo = member_split(om, a.nouter_m, a.mstride);
-    const long long io = outer_index(om, a.outer_keep, a.outer_n);
-    return fl.p[f] + mo + io * a.ostride + (long long)chunk * C + c;
+    const int io = outer_index(om, a.outer_keep, a.outer_n);
+    r = tile_rows(a.sph, io, a.outer_n, chunk * C, box_keep);
+    r.live = r.live && active;
+    return fl.p[f] + mo + (long long)io * a.ostride + (long long)chunk * C + c;
+  };
+  // with one group per block the removed columns are passed over
+  auto live_from = [&](int tile) {
+    if (a.G == 1 && a.sph.axis == 0) {
+      TileRows r;
+      for (; tile < ntiles; tile += gridDim.x) {
+        (void)base_of(tile, r, -1);
+        if (r.live) break;
+      }
+    }
+    return tile;
   };
   auto load = [&](int tile, cx<T>* v) {
-    bool active;
-    const cx<T>* base = base_of(tile, active);
+    TileRows r;
+    const cx<T>* base = base_of(tile, r, a.in_keep);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = t + e * TPC;
-      v[e] = (active && row_kept(p, L, a.in_keep)) ? ld_s(&base[(long long)p * a.estride]) : mk<T>(0, 0);
+      v[e] = (r.live && row_kept(p, L, r.keep)) ? ld_s(&base[(long long)p * a.estride]) : mk<T>(0, 0);
     }
   };
-  int tile = blockIdx.x;
+  int tile = live_from(blockIdx.x);
+  if (tile >= ntiles) return;
   cx<T> v[E], nv[E];
   load(tile, v);
   // The twiddles are read from a copy in LDS after the G column regions.  Held in registers from
@@ -150,7 +208,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   __syncthreads();
   const LdsCol idx{g * L * C + c, C};
   while (true) {
-    const int next = tile + gridDim.x;
+    const int next = live_from(tile + gridDim.x);
     const bool more = next < ntiles;
     if (more) load(next, nv);
     fft<T, L, SIGN>(v, lds, t, idx, twl);
@@ -160,13 +218,13 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
     // compiler, the wait came after the stores (for the copy of the next tile), exposing their
     // full latency once per tile.
     wait_vmem();
-    bool active;
-    cx<T>* base = base_of(tile, active);
-    if (active) {
+    TileRows r;
+    cx<T>* base = base_of(tile, r, a.out_keep);
+    if (r.live) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int p = t + e * TPC;
-        if (row_kept(p, L, a.out_keep)) st_s(&base[(long long)p * a.estride], v[e]);
+        if (row_kept(p, L, r.keep)) st_s(&base[(long long)p * a.estride], v[e]);
       }
     }
     if (!more) break;

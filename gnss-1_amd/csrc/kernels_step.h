@@ -147,13 +147,8 @@ __global__ void k_rk(Geom g, Box b, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const 
   box_index(g, b, i, ix, iy, iz);
   const long long o = m * c.mstride + ((long long)ix * g.ny + iy) * g.kzs + iz;
   const int mz = mode_of(iz, g.nz);
-  if (iz >= g.nzh || !kept(g, mode_of(ix, g.nx), mode_of(iy, g.ny), mz)) {
-    for (int f = 0; f < F; ++f) {
-      st_s(&q.p[f][o], mk<T>(0, 0));
-      if (!c.last) st_s(&dq.p[f][o], mk<T>(0, 0));
-    }
-    return;
-  }
+  // removed modes: the state holds zeros there (the step starts from a dealiased one)
+  if (iz >= g.nzh || !kept(g, mode_of(ix, g.nx), mode_of(iy, g.ny), mz)) return;
   const T kx = kxv[ix], ky = kyv[iy], kz = kzv[iz];
   const T k2 = kx * kx + ky * ky + kz * kz;
   cx<T> rhs[MAXF];
@@ -712,33 +707,46 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
   const int c = tid % C;
   const int t = (tid / C) % TPC;
   const int g = tid / (C * TPC);
-  auto offset_of = [&](int tile, bool& active, int& iy, int& iz) {
+  auto offset_of = [&](int tile, TileRows& r, int& iy, int& iz) {
     const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;
     const int o = (lt / a.nchunks) * a.G + g;
-    active = o < a.nouter;
+    const bool active = o < a.nouter;
     iy = outer_index(active ? o : 0, a.outer_keep, a.outer_n);
     iz = chunk * C + c;
+    r = tile_rows(a.sph, iy, a.outer_n, chunk * C, a.in_keep);
+    r.live = r.live && active;
     return (long long)iy * a.ostride + iz;
+  };
+  auto live_from = [&](int tile) {
+    if (a.G == 1 && a.sph.axis == 0) {
+      TileRows r;
+      int iy, iz;
+      for (; tile < ntiles; tile += gridDim.x) {
+        (void)offset_of(tile, r, iy, iz);
+        if (r.live) break;
+      }
+    }
+    return tile;
   };
   // A is loaded one tile ahead; B (two-input operation) when the tile is formed, which keeps the
   // register footprint of a 16-column tile without spills
   auto load_col = [&](bool second, int tile, cx<T>* va) {
     const cx<T>* __restrict__ src = second ? li.B[tile / tpf] : li.A[tile / tpf];
-    bool active;
+    TileRows r;
     int iy, iz;
-    const long long off = offset_of(tile, active, iy, iz);
+    const long long off = offset_of(tile, r, iy, iz);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = t + e * TPC;
-      const bool ld = active && row_kept(p, L, a.in_keep);
+      const bool ld = r.live && row_kept(p, L, r.keep);
       va[e] = ld ? ld_s(&src[off + (long long)p * a.estride]) : mk<T>(0, 0);
     }
   };
   auto form = [&](int tile, const cx<T>* va, cx<T>* v) {
-    bool active;
+    TileRows r;
     int iy, iz;
-    (void)offset_of(tile, active, iy, iz);
+    (void)offset_of(tile, r, iy, iz);
     const T ky = kyv[iy], kz = kzv[iz];
     const XOp op = li.op[tile / tpf];
     cx<T> vb[TWO ? E : 1];
@@ -757,20 +765,21 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
       }
     }
   };
-  int tile = blockIdx.x;
+  int tile = live_from(blockIdx.x);
+  if (tile >= ntiles) return;
   cx<T> va[E], v[E];
   load_col(false, tile, va);
   const LdsCol idx{g * L * C + c, C};
   while (true) {
     form(tile, va, v);
-    const int next = tile + gridDim.x;
+    const int next = live_from(tile + gridDim.x);
     const bool more = next < ntiles;
     if (more) load_col(false, next, va);
     fft<T, L, +1>(v, lds, t, idx, tw);
-    bool active;
+    TileRows r;
     int iy, iz;
-    const long long off = offset_of(tile, active, iy, iz);
-    if (active) {
+    const long long off = offset_of(tile, r, iy, iz);
+    if (r.live) {
       cx<T>* __restrict__ out = li.out[tile / tpf];
 #pragma unroll
       for (int e = 0; e < E; ++e) st_s(&out[off + (long long)(t + e * TPC) * a.estride], v[e]);
@@ -814,25 +823,20 @@ constexpr unsigned removed_slabs(int L, int TPC, int E) {
   return m;
 }
 
-// Forms of the two-output kernels: both outputs through the radix stages together in two LDS
-// regions, A loaded with its tile (PAIR_BATCHED); one after the other through one region, the
-// next tile's A loaded once the last output is formed (PAIR_SEQ: half the LDS); together, with the
-// next tile's A loaded before they transform (PAIR_BATCHED_PF).
-constexpr int PAIR_BATCHED = 0, PAIR_SEQ = 1, PAIR_BATCHED_PF = 2;
-
-// Persistent like k_xinv_op_pipe: tile i is tile i % tpf of list entry i / tpf; B is loaded with
-// A (one tile ahead in the prefetching forms).  NIN, NOUT: inputs and outputs of every entry of the
-// launch; FORM: how two outputs share the block (one output: always with the next tile loaded
-// before the transform).
+// Persistent like k_xinv_op_pipe, over the entries of a whole pass: tile i is tile i % tpf of list entry
+// i / tpf, entries of one or two inputs and outputs together (the branches are uniform over the block), so
+// a pass is one launch with one tail.  Two outputs go through the radix stages one after the other in
+// one LDS region; the next tile's inputs are loaded once the last output is formed, ahead of its
+// transform.  Columns of removed modes are passed over and only rows inside the ellipsoid are loaded.
 // The twiddles are read from a copy in LDS, after the data regions: read from memory, each radix
 // stage would wait for every load in flight, the next tile's included.  An entry
 // may write its outputs over its own inputs (each tile is read before it is written, by the one
 // block that owns it, and both outputs are formed from registers); no entry may read a field
 // another entry writes.
-template <typename T, int L, int C, int NIN, int NOUT, int FORM>
+template <typename T, int L, int C>
 __global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
-k_inv_pair_pipe(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ tw, ColArgs a, int tpf,
-                int ntiles) {
+k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ tw, ColArgs a, int tpf,
+           int ntiles) {
   constexpr int E = Plan<L>::E;
   constexpr int TPC = L / E;
   extern __shared__ unsigned char smem_raw[];
@@ -844,62 +848,61 @@ k_inv_pair_pipe(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restric
   // Element (row p = t + e TPC, column c) of a tile sits at tile_off(tile) + e TPC estride (the
   // same for the whole group: with one group per block, wave-uniform) plus the lane's
   // c + t estride, which the host keeps below 2^32 bytes.
-  auto tile_off = [&](int tile, bool& active) {
+  auto tile_off = [&](int tile, TileRows& r) {
     const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;
     const int o = (lt / a.nchunks) * a.G + g;
-    active = o < a.nouter;
+    const bool active = o < a.nouter;
     int om = active ? o : 0;
     const long long mo = member_split(om, a.nouter_m, a.mstride);
     const int io = outer_index(om, a.outer_keep, a.outer_n);
+    r = tile_rows(a.sph, io, a.outer_n, chunk * C, a.in_keep);
+    r.live = r.live && active;
     return mo + (long long)io * a.ostride + chunk * C;
+  };
+  auto live_from = [&](int tile) {
+    if (a.G == 1 && a.sph.axis == 0) {
+      TileRows r;
+      for (; tile < ntiles; tile += gridDim.x) {
+        (void)tile_off(tile, r);
+        if (r.live) break;
+      }
+    }
+    return tile;
   };
   const unsigned lane_b = (unsigned)(c + (long long)t * a.estride) * (unsigned)sizeof(cx<T>);
   // the inputs hold the rows the 2/3 rule keeps (in_keep = L / 3, checked by the host): the slabs
   // of removed rows are zeros known at compile time, neither loaded nor transformed
   constexpr unsigned ZS = removed_slabs(L, TPC, E);
-  auto load_col = [&](const cx<T>* __restrict__ src, int tile, cx<T>* va) {
-    bool active;
-    const long long off = tile_off(tile, active);
+  cx<T> va[E], vb[E];
+  auto load_tile = [&](int tile) {
+    const int ent = tile / tpf;
+    TileRows r;
+    const long long off = tile_off(tile, r);
+    const cx<T>* __restrict__ A = li.A[ent];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int p = t + e * TPC;
-      va[e] = (!((ZS >> e) & 1u) && active && row_kept(p, L, a.in_keep))
-                  ? ld_at(src + off + (long long)e * TPC * a.estride, lane_b)
+    for (int e = 0; e < E; ++e)
+      va[e] = (!((ZS >> e) & 1u) && r.live && row_kept(t + e * TPC, L, r.keep))
+                  ? ld_at(A + off + (long long)e * TPC * a.estride, lane_b)
                   : mk<T>(0, 0);
+    if (li.op[ent].nin == 2) {
+      const cx<T>* __restrict__ B = li.B[ent];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        vb[e] = (!((ZS >> e) & 1u) && r.live && row_kept(t + e * TPC, L, r.keep))
+                    ? ld_at(B + off + (long long)e * TPC * a.estride, lane_b)
+                    : mk<T>(0, 0);
     }
   };
-  constexpr bool SEQ = NOUT == 2 && FORM == PAIR_SEQ;
-  // G groups of C columns; each group owns NREG regions of L x C entries
-  constexpr int NREG = SEQ ? 1 : NOUT;
-  const LdsCol idx{g * NREG * L * C + c, C};
-  constexpr bool PF = NOUT == 1 || FORM != PAIR_BATCHED;
-  // output j of entry op at this thread's positions
+  const LdsCol idx{g * L * C + c, C};
   // the wavenumbers of this thread's rows, loaded once before the loop (see wait_vmem below)
   T kr[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) kr[e] = kv[t + e * TPC];
-  auto form = [&](const PairOp& op, int j, const cx<T>* va, const cx<T>* vb, cx<T>* r) {
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const T k = kr[e];
-      const T ka = (T)op.b[j] * k, ra = (T)op.a[j];
-      cx<T> x = mk<T>(ra * va[e].x - ka * va[e].y, ra * va[e].y + ka * va[e].x);
-      if (NIN == 2) {
-        const T kb = (T)op.d[j] * k, rb = (T)op.c[j];
-        const cx<T> b = vb[NIN == 2 ? e : 0];
-        x.x += rb * b.x - kb * b.y;
-        x.y += rb * b.y + kb * b.x;
-      }
-      r[e] = x;
-    }
-  };
-  int tile = blockIdx.x;
-  // the prefetching forms load the next tile's B with its A
-  cx<T> va[E], vb[NIN == 2 ? E : 1];
-  if (PF) load_col(li.A[tile / tpf], tile, va);
-  if (PF && NIN == 2) load_col(li.B[tile / tpf], tile, vb);
-  cx<T>* twl = lds + (long long)a.G * NREG * L * C;
+  int tile = live_from(blockIdx.x);
+  if (tile >= ntiles) return;
+  load_tile(tile);
+  cx<T>* twl = lds + (long long)a.G * L * C;
   for (int i = tid; i < L; i += blockDim.x) twl[i] = tw[i];
   // Nothing in flight when the loop starts: loads issued on paths that may skip some of them (the
   // copy loop above, lane predicates) leave the compiler unable to count the loads in flight, and
@@ -909,50 +912,40 @@ k_inv_pair_pipe(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restric
   while (true) {
     const int ent = tile / tpf;
     const PairOp op = li.op[ent];
-    if (!PF) load_col(li.A[ent], tile, va);
-    if (!PF && NIN == 2) load_col(li.B[ent], tile, vb);
-    const int next = tile + gridDim.x;
+    const int next = live_from(tile + gridDim.x);
     const bool more = next < ntiles;
-    bool active;
-    const long long off = tile_off(tile, active);
-    if constexpr (SEQ) {
+    TileRows r;
+    const long long off = tile_off(tile, r);
+#pragma unroll 1
+    for (int j = 0; j < op.nout; ++j) {
+      const T ra = (T)(j ? op.a[1] : op.a[0]), ba = (T)(j ? op.b[1] : op.b[0]);
+      const T rb = (T)(j ? op.c[1] : op.c[0]), db = (T)(j ? op.d[1] : op.d[0]);
+      cx<T> v[1][E];
 #pragma unroll
-      for (int j = 0; j < NOUT; ++j) {
-        cx<T> v[1][E];
-        form(op, j, va, vb, v[0]);
-        if (j == NOUT - 1 && more) {
-          load_col(li.A[next / tpf], next, va);
-          if (NIN == 2) load_col(li.B[next / tpf], next, vb);
-        }
-        fft_batch<T, L, +1, LdsCol, Plan<L>, false, 1, L * C>(v, lds, t, idx, twl);
-        // one wait per tile, after its last transform and before its last stores: the counter
-        // covers loads and stores alike, so any wait with both in flight waits for all of them;
-        // here the next tile's loads have had a whole transform to arrive, where the compiler's
-        // own wait came after the stores and exposed their latency once per tile
-        if (j == NOUT - 1) wait_vmem();
-        if (active) {
-          cx<T>* __restrict__ dst = li.out[j][ent];
+      for (int e = 0; e < E; ++e) {
+        const T ka = ba * kr[e];
+        v[0][e] = mk<T>(ra * va[e].x - ka * va[e].y, ra * va[e].y + ka * va[e].x);
+      }
+      if (op.nin == 2) {
 #pragma unroll
-          for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[0][e]);
+        for (int e = 0; e < E; ++e) {
+          const T kb = db * kr[e];
+          v[0][e].x += rb * vb[e].x - kb * vb[e].y;
+          v[0][e].y += rb * vb[e].y + kb * vb[e].x;
         }
       }
-    } else {
-      cx<T> v[NOUT][E];
+      const bool last = j == op.nout - 1;
+      if (last && more) load_tile(next);
+      fft_batch<T, L, +1, LdsCol, Plan<L>, false, 1, L * C>(v, lds, t, idx, twl);
+      // one wait per tile, after its last transform and before its last stores: the counter
+      // covers loads and stores alike, so any wait with both in flight waits for all of them;
+      // here the next tile's loads have had a whole transform to arrive, where the compiler's
+      // own wait came after the stores and exposed their latency once per tile
+      if (last) wait_vmem();
+      if (r.live) {
+        cx<T>* __restrict__ dst = li.out[j][ent];
 #pragma unroll
-      for (int j = 0; j < NOUT; ++j) form(op, j, va, vb, v[j]);
-      if (PF && more) {
-        load_col(li.A[next / tpf], next, va);
-        if (NIN == 2) load_col(li.B[next / tpf], next, vb);
-      }
-      fft_batch<T, L, +1, LdsCol, Plan<L>, false, NOUT, L * C>(v, lds, t, idx, twl);
-      wait_vmem();  // as in the SEQ form
-      if (active) {
-#pragma unroll
-        for (int j = 0; j < NOUT; ++j) {
-          cx<T>* __restrict__ dst = li.out[j][ent];
-#pragma unroll
-          for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[j][e]);
-        }
+        for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[0][e]);
       }
     }
     if (!more) break;
@@ -981,7 +974,7 @@ template <typename T, int L, int C, bool VEL>
 __global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
 k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kxv,
           const T* __restrict__ kyv, const T* __restrict__ kzv, const cx<T>* __restrict__ tw, RkCoef rc,
-          int scalar, int nchunks, int G) {
+          Sphere sph, int scalar, int nchunks, int G) {
   constexpr int NF = VEL ? 3 : 1;
   constexpr int E = Plan<L>::E;
   constexpr int TPC = L / E;
@@ -994,8 +987,10 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
   const int chunk = blockIdx.x % nchunks;
   const int o = (blockIdx.x / nchunks) * G + gg;
   const int nouter = 2 * g.keep_y + 1;
-  const bool active = o < nouter;
-  const int iy = outer_index(active ? o : 0, g.keep_y, g.ny);
+  const int iy = outer_index(o < nouter ? o : 0, g.keep_y, g.ny);
+  // a column of removed modes has no right-hand side, and its state is zero already
+  const bool active = o < nouter && tile_rows(sph, iy, g.ny, chunk * C, g.keep_x).live;
+  if (G == 1 && !active) return;
   const int iz = chunk * C + c;
   const long long estride = (long long)g.ny * g.kzs;
   // element (row p = t + e TPC, column c) at at(e) (wave-uniform with one group per block) plus the
@@ -1089,8 +1084,7 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
     for (int j = 0; j < EB && PRE; ++j) {
       const int p = t + (e0 + j) * TPC;
       const long long o2 = at(e0 + j);
-      const bool live = !((ZS >> (e0 + j)) & 1u) && row_kept(p, L, g.keep_x) && iz < g.nzh &&
-                        kept(g, mode_of(p, g.nx), my, mz);
+      const bool live = !((ZS >> (e0 + j)) & 1u) && iz < g.nzh && kept(g, mode_of(p, g.nx), my, mz);
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         od[j][f] = (live && !rc.first) ? ld_at(dq.p[f0 + f] + o2, lane_b) : mk<T>(0, 0);
@@ -1101,16 +1095,9 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
     for (int j = 0; j < EB; ++j) {
       const int e = e0 + j;
       const int p = t + e * TPC;
-      if (((ZS >> e) & 1u) || !row_kept(p, L, g.keep_x)) continue;
+      // removed modes: the state holds zeros there (the step starts from a dealiased one)
+      if (((ZS >> e) & 1u) || iz >= g.nzh || !kept(g, mode_of(p, g.nx), my, mz)) continue;
       const long long o2 = at(e);
-      if (iz >= g.nzh || !kept(g, mode_of(p, g.nx), my, mz)) {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          st_at(q.p[f0 + f] + o2, lane_b, mk<T>(0, 0));
-          if (!rc.last) st_at(dq.p[f0 + f] + o2, lane_b, mk<T>(0, 0));
-        }
-        continue;
-      }
       const T kx = kxl[p];
       const T k2 = kx * kx + ky * ky + kz * kz;
       cx<T> rhs[NF];
