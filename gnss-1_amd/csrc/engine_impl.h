@@ -180,6 +180,7 @@ class Engine : public EngineBase {
     if (nb_ > 1) select_member(0);
     t_ = 0;
     step_ = 0;
+    clean_ = true;  // build_initial_condition leaves the removed modes out
     have_ic_ = true;
   }
   void init_jet_member() {
@@ -211,14 +212,14 @@ class Engine : public EngineBase {
 
   void forward(int f) override {
     check_field(f);
+    clean_ = false;
     fwd3d(phys_[f], q_[f], false);
     sync();
   }
 
   void inverse(int f) override {
     check_field(f);
-    GNSS_HIP(hipMemcpyAsync(ws_[0], q_[f], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
-    inv3d(ws_[0], phys_[f], false);
+    state_to_physical(f, 1, &phys_[f]);
     sync();
   }
 
@@ -226,6 +227,7 @@ class Engine : public EngineBase {
     need_k();
     hipLaunchKernelGGL(k_dealias<T>, dim3(cdiv(nsp_, 256)), dim3(256), 0, s_, g_, ptrs(q_), F_, nsp_);
     check_launch("k_dealias");
+    clean_ = true;
     sync();
   }
 
@@ -234,13 +236,15 @@ class Engine : public EngineBase {
     if (nsteps < 0) throw Error(GNSS_ERR_ARG, "nsteps must be >= 0");
     if (nsteps == 0) return;
     // the step starts from a dealiased state (deAlias at the top of solver_ps, solver.cu:704);
-    // every substage keeps it dealiased afterwards
-    for (int m = 0; m < nb_; ++m) {
-      if (nb_ > 1) select_member(m);
-      timed("k_dealias", (double)nsp_ * F_ * sizeof(C), [&] {
-        hipLaunchKernelGGL(k_dealias<T>, dim3(cdiv(nsp_, 256)), dim3(256), 0, s_, g_, ptrs(q_), F_, nsp_);
-      });
-    }
+    // every substage keeps it dealiased afterwards, so only a state written from outside needs it
+    if (!clean_)
+      for (int m = 0; m < nb_; ++m) {
+        if (nb_ > 1) select_member(m);
+        timed("k_dealias", (double)nsp_ * F_ * sizeof(C), [&] {
+          hipLaunchKernelGGL(k_dealias<T>, dim3(cdiv(nsp_, 256)), dim3(256), 0, s_, g_, ptrs(q_), F_, nsp_);
+        });
+      }
+    clean_ = true;
     for (int n = 0; n < nsteps; ++n) enqueue_rk3_step();
     advance_clock(nsteps);
     check_finite();
@@ -377,10 +381,7 @@ class Engine : public EngineBase {
         hipLaunchKernelGGL(k_spectrum<T>, dim3(nx_), dim3(STAT_THREADS), 0, s_, g_, ptrs(q_), S_, nb, sa,
                            inn2, spec);
       });
-    for (int f = 0; f < F_; ++f) {
-      GNSS_HIP(hipMemcpyAsync(ws_[0], q_[f], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
-      inv3d(ws_[0], phys_[f], false);
-    }
+    state_to_physical(0, F_, phys_.data());
     RPtrs<T> pp{};
     for (int f = 0; f < F_; ++f) pp.p[f] = phys_[f];
     timed("k_plane_stats", (double)F_ * nph_ * sizeof(T), [&] {
@@ -447,6 +448,7 @@ class Engine : public EngineBase {
       return;
     }
     if (space != GNSS_SPECTRAL) throw Error(GNSS_ERR_ARG, "bad space");
+    clean_ = false;
     std::vector<C> h(nsp_);
     memset((void*)h.data(), 0, sizeof(C) * nsp_);
     for (int y = 0; y < ny_; ++y)
@@ -505,14 +507,13 @@ class Engine : public EngineBase {
     GNSS_HIP(hipEventCreate(&e1));
     GNSS_HIP(hipEventCreate(&e2));
     // warm-up pair
-    inv3d_keep(q_[0], ws_[0], phys_[0]);
+    const C* spec = q_[0];
+    inv3d(&spec, ws_.data(), phys_.data(), 1, false);
     fwd3d(phys_[0], ws_[1], false);
     float tf = 0, ti = 0;
     for (int r = 0; r < reps; ++r) {
-      GNSS_HIP(hipEventRecord(e0, s_));
-      GNSS_HIP(hipMemcpyAsync(ws_[0], q_[0], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
       GNSS_HIP(hipEventRecord(e1, s_));
-      inv3d(ws_[0], phys_[0], false);
+      inv3d(&spec, ws_.data(), phys_.data(), 1, false);
       GNSS_HIP(hipEventRecord(e2, s_));
       GNSS_HIP(hipEventSynchronize(e2));
       float a = 0, b = 0;
@@ -597,14 +598,15 @@ class Engine : public EngineBase {
     T* out;
     if (field >= 0) {
       out = reinterpret_cast<T*>(ws_[1]);
-      GNSS_HIP(hipMemcpyAsync(ws_[0], q_[field], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
-      inv3d(ws_[0], out, false);
+      state_to_physical(field, 1, &out);
     } else {
       CPtrs<T> w{};
       for (int c = 0; c < 3; ++c) w.p[c] = ws_[c];
       hipLaunchKernelGGL(k_vorticity<T>, dim3((unsigned)cdiv(nsp_, 256)), dim3(256), 0, s_, g_, ptrs(q_), w, tkx_,
                          tky_, tkz_, nsp_);
-      for (int c = 0; c < 3; ++c) inv3d(ws_[c], reinterpret_cast<T*>(ws_[3 + c]), false);
+      T* om[3];
+      for (int c = 0; c < 3; ++c) om[c] = reinterpret_cast<T*>(ws_[3 + c]);
+      inv3d(ws_.data(), ws_.data(), om, 3, clean_);
       out = reinterpret_cast<T*>(ws_[3]);
       hipLaunchKernelGGL(k_magnitude<T>, dim3((unsigned)cdiv(nph_, 256)), dim3(256), 0, s_, out,
                          reinterpret_cast<const T*>(ws_[4]), reinterpret_cast<const T*>(ws_[5]), nph_);
@@ -1156,7 +1158,7 @@ class Engine : public EngineBase {
 
   // the pass over nf fields: persistent blocks over all their tiles (cp), else one launch per field
   template <int L, int SIGN, int CC>
-  void col_launch(C* const* fields, int nf, const ColArgs& a, int G) {
+  void col_launch(const FieldList<T>& fl, int nf, const ColArgs& a, int G) {
     constexpr int TPC = L / Plan<L>::E;
     const int threads = CC * TPC * G;
     const size_t lds = (size_t)G * L * CC * sizeof(C);
@@ -1168,19 +1170,15 @@ class Engine : public EngineBase {
       const long long per_cu = std::max<long long>(1, std::min<long long>(160 * 1024 / (long long)ldsp,
                                                                            2048 / threads));
       const long long grid = std::min<long long>(blocks * nf, per_cu * n_cu_);
-      FieldList<T> fl{};
-      for (int f = 0; f < nf; ++f) fl.p[f] = fields[f];
       hipLaunchKernelGGL((k_col_multi<T, L, SIGN, CC>), dim3((unsigned)grid), dim3(threads), ldsp, s_, fl,
                          tw_.at(L), a, (int)blocks, (int)(blocks * nf));
       return;
     }
-    for (int f = 0; f < nf; ++f)
-      hipLaunchKernelGGL((k_col<T, L, SIGN, CC>), dim3((unsigned)blocks), dim3(threads), lds, s_, fields[f],
-                         tw_.at(L), a);
+    hipLaunchKernelGGL((k_col<T, L, SIGN, CC>), dim3((unsigned)blocks, nf), dim3(threads), lds, s_, fl, tw_.at(L), a);
   }
 
   template <int L, int SIGN>
-  void col_dispatch_c(C* const* fields, int nf, const ColArgs& a, int CC, int G) {
+  void col_dispatch_c(const FieldList<T>& fields, int nf, const ColArgs& a, int CC, int G) {
     if constexpr (sizeof(T) == 8) {
       if (CC == 8) col_launch<L, SIGN, 8>(fields, nf, a, G);
       else col_launch<L, SIGN, 4>(fields, nf, a, G);
@@ -1195,24 +1193,24 @@ class Engine : public EngineBase {
     return sizeof(T) == 4 && (p_.flags & GNSS_FLAG_MFMA_R16) && (L == 256 || L == 512 || L == 1024);
   }
   template <int L, int SIGN, int CC>
-  void mfma_launch(C* data, const ColArgs& a) {
+  void mfma_launch(const C* in, C* out, const ColArgs& a) {
     if constexpr (sizeof(T) == 4) {
       const size_t lds = (size_t)L * CC * sizeof(C);
       const long long blocks = (long long)a.nchunks * a.nouter;
       hipLaunchKernelGGL((k_col_mfma<L, SIGN, CC>), dim3((unsigned)blocks), dim3(CC * (L / 16)), lds, s_,
-                         data, tw_.at(L), a);
+                         in, out, tw_.at(L), a);
     }
   }
   template <int SIGN>
-  void mfma_dispatch(int L, C* data, const ColArgs& a, int CC) {
-    if (L == 1024) return mfma_launch<1024, SIGN, 8>(data, a);
-    if (L == 512) return CC == 16 ? mfma_launch<512, SIGN, 16>(data, a) : mfma_launch<512, SIGN, 8>(data, a);
-    if (L == 256) return CC == 16 ? mfma_launch<256, SIGN, 16>(data, a) : mfma_launch<256, SIGN, 8>(data, a);
+  void mfma_dispatch(int L, const C* in, C* out, const ColArgs& a, int CC) {
+    if (L == 1024) return mfma_launch<1024, SIGN, 8>(in, out, a);
+    if (L == 512) return CC == 16 ? mfma_launch<512, SIGN, 16>(in, out, a) : mfma_launch<512, SIGN, 8>(in, out, a);
+    if (L == 256) return CC == 16 ? mfma_launch<256, SIGN, 16>(in, out, a) : mfma_launch<256, SIGN, 8>(in, out, a);
     throw Error(GNSS_ERR_UNSUPPORTED, "MFMA radix-16 stage needs length 256, 512 or 1024");
   }
 
   template <int SIGN>
-  void col_dispatch_l(int L, C* const* data, int nf, const ColArgs& a, int CC, int G) {
+  void col_dispatch_l(int L, const FieldList<T>& data, int nf, const ColArgs& a, int CC, int G) {
     switch (L) {
       case 16: col_dispatch_c<16, SIGN>(data, nf, a, CC, G); break;
       case 24: col_dispatch_c<24, SIGN>(data, nf, a, CC, G); break;
@@ -1252,8 +1250,9 @@ class Engine : public EngineBase {
 
   void col_pass(C* data, const ColSpec& sp) { col_passes(&data, 1, sp); }
 
-  // The same strided pass over nf fields; with cb (and cp) one persistent launch covers them all.
-  void col_passes(C* const* fields, int nf, const ColSpec& sp) {
+  // The same strided pass over nf fields (with cb one launch covers them all), in place or from `in`.
+  void col_passes(C* const* fields, int nf, const ColSpec& sp) { col_passes(fields, fields, nf, sp); }
+  void col_passes(const C* const* in, C* const* fields, int nf, const ColSpec& sp) {
     const int L = sp.axis == 0 ? nx_ : ny_;
     const int CC = sp.axis == 0 ? cx_ : cy_;
     const int TPC = L / elems_per_thread(L);
@@ -1289,17 +1288,23 @@ class Engine : public EngineBase {
                                        : (sp.sign < 0 ? "fft_y_fwd_mfma" : "fft_y_inv_mfma");
       for (int f = 0; f < nf; ++f)
         timed(mname, bytes, [&] {
-          if (sp.sign < 0) mfma_dispatch<-1>(L, fields[f], a, CC);
-          else mfma_dispatch<+1>(L, fields[f], a, CC);
+          if (sp.sign < 0) mfma_dispatch<-1>(L, in[f], fields[f], a, CC);
+          else mfma_dispatch<+1>(L, in[f], fields[f], a, CC);
         });
       return;
     }
     const int groups = cb_ ? 1 : nf, per = cb_ ? nf : 1;
-    for (int gi = 0; gi < groups; ++gi)
+    for (int gi = 0; gi < groups; ++gi) {
+      FieldList<T> fl{};
+      for (int f = 0; f < per; ++f) {
+        fl.in[f] = in[gi * per + f];
+        fl.p[f] = fields[gi * per + f];
+      }
       timed(name, bytes * per, [&] {
-        if (sp.sign < 0) col_dispatch_l<-1>(L, fields + gi * per, per, a, CC, G);
-        else col_dispatch_l<+1>(L, fields + gi * per, per, a, CC, G);
+        if (sp.sign < 0) col_dispatch_l<-1>(L, fl, per, a, CC, G);
+        else col_dispatch_l<+1>(L, fl, per, a, CC, G);
       });
+    }
   }
 
   template <int NZ>
@@ -1321,7 +1326,7 @@ class Engine : public EngineBase {
                        tw_.at(M), tw_.at(NZ), rows, kzs_, out_lim, G);
   }
   template <int NZ>
-  void zc2r_launch(const C* in, T* out, int in_lim, T scale) {
+  void zc2r_launch(const ZList<T>& zl, int nf, int in_lim, T scale) {
     constexpr int M = NZ / 2;
     constexpr int TPC = M / Plan<M>::E;
     int G = std::max(1, 256 / TPC);
@@ -1331,13 +1336,13 @@ class Engine : public EngineBase {
     if (zp_) {
       const long long groups = cdiv(rows, G);
       const size_t ldsp = lds + 2 * (size_t)M * sizeof(C);  // and both twiddle tables
-      hipLaunchKernelGGL((k_c2r_z_pipe<T, NZ>), dim3((unsigned)std::min(groups, zpipe_blocks(ldsp, TPC * G))),
-                         dim3(TPC * G), ldsp, s_, in, out, tw_.at(M), tw_.at(NZ), rows, kzs_, in_lim, scale, G,
-                         groups);
+      const long long resident = std::max<long long>(1, cdiv(zpipe_blocks(ldsp, TPC * G), nf));
+      hipLaunchKernelGGL((k_c2r_z_pipe<T, NZ>), dim3((unsigned)std::min(groups, resident), nf), dim3(TPC * G), ldsp,
+                         s_, zl, tw_.at(M), tw_.at(NZ), rows, kzs_, in_lim, scale, G, groups);
       return;
     }
-    hipLaunchKernelGGL((k_c2r_z<T, NZ>), dim3((unsigned)cdiv(rows, G)), dim3(TPC * G), lds, s_, in, out,
-                       tw_.at(M), tw_.at(NZ), rows, kzs_, in_lim, scale, G);
+    hipLaunchKernelGGL((k_c2r_z<T, NZ>), dim3((unsigned)cdiv(rows, G), nf), dim3(TPC * G), lds, s_, zl, tw_.at(M),
+                       tw_.at(NZ), rows, kzs_, in_lim, scale, G);
   }
 
   // blocks of a persistent z pass: as many as stay resident on every CU (LDS and wave limits)
@@ -1368,9 +1373,15 @@ class Engine : public EngineBase {
     const double bytes = (double)nx_ * ny_ * ((double)nz_ * sizeof(T) + (double)std::min(out_lim, kzs_) * sizeof(C));
     timed("fft_z_r2c", bytes, [&] { GNSS_Z_SWITCH(zr2c_launch, in, out, out_lim); });
   }
-  void z_c2r(const C* in, T* out, int in_lim, T scale) {
-    const double bytes = (double)nx_ * ny_ * ((double)nz_ * sizeof(T) + (double)std::min(in_lim, nzh_) * sizeof(C));
-    timed("fft_z_c2r", bytes, [&] { GNSS_Z_SWITCH(zc2r_launch, in, out, in_lim, scale); });
+  void z_c2r(const C* in, T* out, int in_lim, T scale) { z_c2r(&in, &out, 1, in_lim, scale); }
+  void z_c2r(const C* const* in, T* const* out, int nf, int in_lim, T scale) {
+    ZList<T> zl{};
+    for (int f = 0; f < nf; ++f) {
+      zl.in[f] = in[f];
+      zl.out[f] = out[f];
+    }
+    const double bytes = (double)nf * nx_ * ny_ * ((double)nz_ * sizeof(T) + (double)std::min(in_lim, nzh_) * sizeof(C));
+    timed("fft_z_c2r", bytes, [&] { GNSS_Z_SWITCH(zc2r_launch, zl, nf, in_lim, scale); });
   }
 
   // Forward 3D R2C: in (physical) -> out (spectral).  prune: only the kept box is produced.
@@ -1386,24 +1397,27 @@ class Engine : public EngineBase {
     col_pass(out, ColSpec{0, -1, kz_lim_ / cx_, g_.keep_y, -1, g_.keep_x});
   }
 
-  // Inverse 3D C2R with 1/(nx ny nz): spec is overwritten (used as the work buffer).
-  void inv3d(C* spec, T* out, bool prune) {
+  // Inverse 3D C2R with 1/(nx ny nz) of nf <= MAXF fields, each pass one launch over all of them.  The
+  // first pass reads spec[f] and writes work[f] (which may be spec[f]); out[f] may not be work[f].
+  // prune: the spectra are zero outside the 2/3 rule's modes, so only those columns and rows are
+  // read (the skipped ones are zeros).  Whole spectra go through y first: the pass that reads one array
+  // and writes another is cheaper along y (512^3 FP32: 0.19 ms) than along x, where every row of a tile
+  // is a page of its own in both (0.30 ms, 0.23 ms in place).
+  void inv3d(const C* const* spec, C* const* work, T* const* out, int nf, bool prune) {
     const T scale = (T)(1.0 / ((double)nx_ * ny_ * nz_));
     if (!prune) {
-      col_pass(spec, ColSpec{0, +1, kzs_ / cx_, -1, -1, -1});
-      col_pass(spec, ColSpec{1, +1, kzs_ / cy_, -1, -1, -1});
-      z_c2r(spec, out, nzh_, scale);
+      col_passes(spec, work, nf, ColSpec{1, +1, kzs_ / cy_, -1, -1, -1});
+      col_passes(work, nf, ColSpec{0, +1, kzs_ / cx_, -1, -1, -1});
+      z_c2r(work, out, nf, nzh_, scale);
       return;
     }
-    col_pass(spec, ColSpec{0, +1, kz_lim_ / cx_, g_.keep_y, g_.keep_x, -1});
-    col_pass(spec, ColSpec{1, +1, kz_lim_ / cy_, -1, g_.keep_y, -1});
-    z_c2r(spec, out, kz_lim_, scale);
+    col_passes(spec, work, nf, ColSpec{0, +1, kz_lim_ / cx_, g_.keep_y, g_.keep_x, -1});
+    col_passes(work, nf, ColSpec{1, +1, kz_lim_ / cy_, -1, g_.keep_y, -1});
+    z_c2r(work, out, nf, kz_lim_, scale);
   }
-
-  void inv3d_keep(const C* spec, C* work, T* out) {
-    GNSS_HIP(hipMemcpyAsync(work, spec, sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
-    inv3d(work, out, false);
-  }
+  void inv3d(C* spec, T* out, bool prune) { inv3d(&spec, &spec, &out, 1, prune); }
+  // the state's fields f0 .. f0 + nf - 1, left as they are
+  void state_to_physical(int f0, int nf, T* const* out) { inv3d(q_.data() + f0, ws_.data(), out, nf, clean_); }
 
   // -------------------------------------------------------------------------------------------
   // One RK3 substage: nonlinear terms of the current state, then the IF-RK update.
@@ -1903,6 +1917,9 @@ class Engine : public EngineBase {
   size_t scratch_n_ = 0;
   std::vector<void*> allocs_;
   bool have_k_ = false, have_ic_ = false, pause_timer_ = false;
+  // the state holds no mode that the 2/3 rule removes: false from the moment something other than a
+  // step, the initial condition or dealias() writes it
+  bool clean_ = true;
   double t_ = 0;
   int64_t step_ = 0;
   KernelTimer timer_;

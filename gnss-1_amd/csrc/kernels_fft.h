@@ -104,9 +104,17 @@ __device__ __forceinline__ TileRows tile_rows(const Sphere& s, int outer, int ou
 // Largest block a pass launches: one transform group, or 256 threads of several groups.
 constexpr int lb_threads(int per_group) { return per_group > 256 ? per_group : 256; }
 
+// Fields of a pass: each tile is read from in[f] and written to p[f], which may be the same array (every
+// block reads its whole tile before it writes).
+template <typename T> struct FieldList {
+  const cx<T>* in[MAXW];
+  cx<T>* p[MAXW];
+};
+
+// One block per tile, field blockIdx.y.
 template <typename T, int L, int SIGN, int C>
 __global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
-k_col(cx<T>* __restrict__ data, const cx<T>* __restrict__ tw, ColArgs a) {
+k_col(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a) {
   constexpr int E = Plan<L>::E;
   constexpr int TPC = L / E;
   extern __shared__ unsigned char smem_raw[];
@@ -124,12 +132,14 @@ k_col(cx<T>* __restrict__ data, const cx<T>* __restrict__ tw, ColArgs a) {
   const TileRows in = tile_rows(a.sph, io, a.outer_n, chunk * C, a.in_keep);
   active = active && in.live;
   if (a.G == 1 && !active) return;
-  cx<T>* base = data + mo + (long long)io * a.ostride + (long long)chunk * C + c;
+  const long long off = mo + (long long)io * a.ostride + (long long)chunk * C + c;
+  const cx<T>* src = fl.in[blockIdx.y] + off;
+  cx<T>* base = fl.p[blockIdx.y] + off;
   cx<T> v[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = t + e * TPC;
-    if (active && row_kept(p, L, in.keep)) v[e] = ld_s(&base[(long long)p * a.estride]);
+    if (active && row_kept(p, L, in.keep)) v[e] = ld_s(&src[(long long)p * a.estride]);
     else v[e] = mk<T>(0, 0);
   }
   fft<T, L, SIGN>(v, lds, t, LdsCol{g * L * C + c, C}, tw);
@@ -147,10 +157,6 @@ k_col(cx<T>* __restrict__ data, const cx<T>* __restrict__ tw, ColArgs a) {
 // transforming the current one (stage barriers wait only for LDS traffic, so the loads stay in
 // flight).  Tile i of the launch is tile i % tpf of field i / tpf: the fields of a pass share one
 // launch gap and one tail.
-template <typename T> struct FieldList {
-  cx<T>* p[MAXW];
-};
-
 template <typename T, int L, int SIGN, int C>
 __global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
 k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, int ntiles) {
@@ -162,8 +168,8 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   const int c = tid % C;
   const int t = (tid / C) % TPC;
   const int g = tid / (C * TPC);
-  auto base_of = [&](int tile, TileRows& r, int box_keep) {
-    const int f = tile / tpf, lt = tile % tpf;
+  auto off_of = [&](int tile, TileRows& r, int box_keep) {
+    const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;
     const int o = (lt / a.nchunks) * a.G + g;
     const bool active = o < a.nouter;
@@ -172,14 +178,14 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
     const int io = outer_index(om, a.outer_keep, a.outer_n);
     r = tile_rows(a.sph, io, a.outer_n, chunk * C, box_keep);
     r.live = r.live && active;
-    return fl.p[f] + mo + (long long)io * a.ostride + (long long)chunk * C + c;
+    return mo + (long long)io * a.ostride + (long long)chunk * C + c;
   };
   // with one group per block the removed columns are passed over
   auto live_from = [&](int tile) {
     if (a.G == 1 && a.sph.axis == 0) {
       TileRows r;
       for (; tile < ntiles; tile += gridDim.x) {
-        (void)base_of(tile, r, -1);
+        (void)off_of(tile, r, -1);
         if (r.live) break;
       }
     }
@@ -187,7 +193,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   };
   auto load = [&](int tile, cx<T>* v) {
     TileRows r;
-    const cx<T>* base = base_of(tile, r, a.in_keep);
+    const cx<T>* base = fl.in[tile / tpf] + off_of(tile, r, a.in_keep);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = t + e * TPC;
@@ -219,7 +225,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
     // full latency once per tile.
     wait_vmem();
     TileRows r;
-    cx<T>* base = base_of(tile, r, a.out_keep);
+    cx<T>* base = fl.p[tile / tpf] + off_of(tile, r, a.out_keep);
     if (r.live) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
@@ -445,13 +451,21 @@ k_r2c_z(const T* __restrict__ in, cx<T>* __restrict__ out, const cx<T>* __restri
   Z::template r2c<1>(v, dst, active, out_lim, kzs, lds, LdsRow{g * Z::RS}, t, twM, twN);
 }
 
+// Rows of several fields through one z pass: field blockIdx.y.
+template <typename T> struct ZList {
+  const cx<T>* in[MAXF];
+  T* out[MAXF];
+};
+
 // C2R along contiguous z rows: in = rows of kzs complex (entries kz >= in_lim are treated as 0;
 // imaginary parts of kz = 0 and kz = nz/2 are ignored), out = rows of NZ reals times `scale`.
 template <typename T, int NZ>
 __global__ void __launch_bounds__(lb_threads((NZ / 2) / Plan<NZ / 2>::E))
-k_c2r_z(const cx<T>* __restrict__ in, T* __restrict__ out, const cx<T>* __restrict__ twM,
-        const cx<T>* __restrict__ twN, long long nrows, int kzs, int in_lim, T scale, int G) {
+k_c2r_z(ZList<T> zl, const cx<T>* __restrict__ twM, const cx<T>* __restrict__ twN, long long nrows, int kzs,
+        int in_lim, T scale, int G) {
   using Z = ZRow<T, NZ, Plan<NZ / 2>>;
+  const cx<T>* __restrict__ in = zl.in[blockIdx.y];
+  T* __restrict__ out = zl.out[blockIdx.y];
   extern __shared__ unsigned char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int t = threadIdx.x % Z::TPC;
@@ -523,10 +537,11 @@ k_r2c_z_pipe(const T* __restrict__ in, cx<T>* __restrict__ out, const cx<T>* __r
 
 template <typename T, int NZ>
 __global__ void __launch_bounds__(lb_threads((NZ / 2) / Plan<NZ / 2>::E))
-k_c2r_z_pipe(const cx<T>* __restrict__ in, T* __restrict__ out, const cx<T>* __restrict__ twM,
-             const cx<T>* __restrict__ twN, long long nrows, int kzs, int in_lim, T scale, int G,
-             long long ngroups) {
+k_c2r_z_pipe(ZList<T> zl, const cx<T>* __restrict__ twM, const cx<T>* __restrict__ twN, long long nrows, int kzs,
+             int in_lim, T scale, int G, long long ngroups) {
   using Z = ZRow<T, NZ, Plan<NZ / 2>>;
+  const cx<T>* __restrict__ in = zl.in[blockIdx.y];
+  T* __restrict__ out = zl.out[blockIdx.y];
   extern __shared__ unsigned char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int t = threadIdx.x % Z::TPC;

@@ -45,7 +45,7 @@ __device__ __forceinline__ void cs16(int j, float& c, float& s) {
 
 template <int L, int SIGN, int C>
 __global__ void __launch_bounds__(C * (L / 16))
-k_col_mfma(cx<float>* __restrict__ data, const cx<float>* __restrict__ tw, ColArgs a) {
+k_col_mfma(const cx<float>* in, cx<float>* out, const cx<float>* __restrict__ tw, ColArgs a) {
   constexpr int E = 16;
   constexpr int TPC = L / E;       // threads per column; also the number of radix-16 butterflies
   constexpr int NT = C * TPC;      // threads per block
@@ -60,12 +60,14 @@ k_col_mfma(cx<float>* __restrict__ data, const cx<float>* __restrict__ tw, ColAr
   const int chunk = blockIdx.x % a.nchunks;
   const int o = blockIdx.x / a.nchunks;  // one outer index per block (G = 1)
   const long long io = outer_index(o, a.outer_keep, a.outer_n);
-  cx<float>* base = data + io * a.ostride + (long long)chunk * C + c;
+  const long long off = io * a.ostride + (long long)chunk * C + c;
+  const cx<float>* src = in + off;
+  cx<float>* base = out + off;  // may be the input: every row is read before the first is written
   // 1. coalesced load into the LDS tile [pos][C]
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int p = t + e * TPC;
-    lds[p * C + c] = row_kept(p, L, a.in_keep) ? base[(long long)p * a.estride] : mk<float>(0, 0);
+    lds[p * C + c] = row_kept(p, L, a.in_keep) ? src[(long long)p * a.estride] : mk<float>(0, 0);
   }
   // 2. constant operand: lane row m of the 32 x 32 block matrix, its 16 K entries (hi, lo)
   const int lane = tid & 63;
