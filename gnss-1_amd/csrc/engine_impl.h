@@ -1158,14 +1158,18 @@ class Engine : public EngineBase {
 
   // the pass over nf fields: persistent blocks over all their tiles (cp), else one launch per field
   template <int L, int SIGN, int CC>
-  void col_launch(const FieldList<T>& fl, int nf, const ColArgs& a, int G) {
-    constexpr int TPC = L / Plan<L>::E;
-    const int threads = CC * TPC * G;
-    const size_t lds = (size_t)G * L * CC * sizeof(C);
-    const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
-    if (cp_) {
-      // the persistent form also holds the twiddle table in LDS, after the data regions
-      const size_t ldsp = lds + (size_t)L * sizeof(C);
+  void col_launch(const FieldList<T>& fl, int nf, const ColArgs& a, int G, int axis) {
+    // both forms hold the twiddle table in LDS, after the data regions
+    const size_t lds = ((size_t)G * L * CC + L) * sizeof(C);
+    // Persistent for x passes with cp only: their rows lie a page apart, and one block that loads ahead has
+    // fewer of them open (512^3, whole arrays: FP32 0.24 against 0.25 ms, FP64 0.48 against 0.51); along y
+    // two blocks per CU win at every size (forward pass of a substage at 512^3: FP32 0.43 against 0.48 ms,
+    // FP64 0.85 against 0.88; at 256^3 0.057 against 0.068 and 0.119 against 0.145).
+    if (cp_ && axis == 0) {
+      constexpr int TPC = L / Plan<L>::E;
+      const int threads = CC * TPC * G;
+      const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
+      const size_t ldsp = lds;
       // persistent: as many blocks as stay resident (LDS and wave limits of a CU), all CUs
       const long long per_cu = std::max<long long>(1, std::min<long long>(160 * 1024 / (long long)ldsp,
                                                                            2048 / threads));
@@ -1174,17 +1178,20 @@ class Engine : public EngineBase {
                          tw_.at(L), a, (int)blocks, (int)(blocks * nf));
       return;
     }
-    hipLaunchKernelGGL((k_col<T, L, SIGN, CC>), dim3((unsigned)blocks, nf), dim3(threads), lds, s_, fl, tw_.at(L), a);
+    constexpr int TPC = L / ColPlan<T, L>::E;
+    const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
+    hipLaunchKernelGGL((k_col<T, L, SIGN, CC>), dim3((unsigned)blocks, nf), dim3(CC * TPC * G), lds, s_, fl, tw_.at(L),
+                       a);
   }
 
   template <int L, int SIGN>
-  void col_dispatch_c(const FieldList<T>& fields, int nf, const ColArgs& a, int CC, int G) {
+  void col_dispatch_c(const FieldList<T>& fields, int nf, const ColArgs& a, int CC, int G, int axis) {
     if constexpr (sizeof(T) == 8) {
-      if (CC == 8) col_launch<L, SIGN, 8>(fields, nf, a, G);
-      else col_launch<L, SIGN, 4>(fields, nf, a, G);
+      if (CC == 8) col_launch<L, SIGN, 8>(fields, nf, a, G, axis);
+      else col_launch<L, SIGN, 4>(fields, nf, a, G, axis);
     } else {
-      if (CC == 16) col_launch<L, SIGN, 16>(fields, nf, a, G);
-      else col_launch<L, SIGN, 8>(fields, nf, a, G);
+      if (CC == 16) col_launch<L, SIGN, 16>(fields, nf, a, G, axis);
+      else col_launch<L, SIGN, 8>(fields, nf, a, G, axis);
     }
   }
 
@@ -1210,20 +1217,20 @@ class Engine : public EngineBase {
   }
 
   template <int SIGN>
-  void col_dispatch_l(int L, const FieldList<T>& data, int nf, const ColArgs& a, int CC, int G) {
+  void col_dispatch_l(int L, const FieldList<T>& data, int nf, const ColArgs& a, int CC, int G, int axis) {
     switch (L) {
-      case 16: col_dispatch_c<16, SIGN>(data, nf, a, CC, G); break;
-      case 24: col_dispatch_c<24, SIGN>(data, nf, a, CC, G); break;
-      case 32: col_dispatch_c<32, SIGN>(data, nf, a, CC, G); break;
-      case 48: col_dispatch_c<48, SIGN>(data, nf, a, CC, G); break;
-      case 64: col_dispatch_c<64, SIGN>(data, nf, a, CC, G); break;
-      case 96: col_dispatch_c<96, SIGN>(data, nf, a, CC, G); break;
-      case 128: col_dispatch_c<128, SIGN>(data, nf, a, CC, G); break;
-      case 192: col_dispatch_c<192, SIGN>(data, nf, a, CC, G); break;
-      case 256: col_dispatch_c<256, SIGN>(data, nf, a, CC, G); break;
-      case 384: col_dispatch_c<384, SIGN>(data, nf, a, CC, G); break;
-      case 512: col_dispatch_c<512, SIGN>(data, nf, a, CC, G); break;
-      case 1024: col_dispatch_c<1024, SIGN>(data, nf, a, CC, G); break;
+      case 16: col_dispatch_c<16, SIGN>(data, nf, a, CC, G, axis); break;
+      case 24: col_dispatch_c<24, SIGN>(data, nf, a, CC, G, axis); break;
+      case 32: col_dispatch_c<32, SIGN>(data, nf, a, CC, G, axis); break;
+      case 48: col_dispatch_c<48, SIGN>(data, nf, a, CC, G, axis); break;
+      case 64: col_dispatch_c<64, SIGN>(data, nf, a, CC, G, axis); break;
+      case 96: col_dispatch_c<96, SIGN>(data, nf, a, CC, G, axis); break;
+      case 128: col_dispatch_c<128, SIGN>(data, nf, a, CC, G, axis); break;
+      case 192: col_dispatch_c<192, SIGN>(data, nf, a, CC, G, axis); break;
+      case 256: col_dispatch_c<256, SIGN>(data, nf, a, CC, G, axis); break;
+      case 384: col_dispatch_c<384, SIGN>(data, nf, a, CC, G, axis); break;
+      case 512: col_dispatch_c<512, SIGN>(data, nf, a, CC, G, axis); break;
+      case 1024: col_dispatch_c<1024, SIGN>(data, nf, a, CC, G, axis); break;
       default: throw Error(GNSS_ERR_UNSUPPORTED, "unsupported transform length " + std::to_string(L));
     }
   }
@@ -1301,8 +1308,8 @@ class Engine : public EngineBase {
         fl.p[f] = fields[gi * per + f];
       }
       timed(name, bytes * per, [&] {
-        if (sp.sign < 0) col_dispatch_l<-1>(L, fl, per, a, CC, G);
-        else col_dispatch_l<+1>(L, fl, per, a, CC, G);
+        if (sp.sign < 0) col_dispatch_l<-1>(L, fl, per, a, CC, G, sp.axis);
+        else col_dispatch_l<+1>(L, fl, per, a, CC, G, sp.axis);
       });
     }
   }
@@ -1651,25 +1658,21 @@ class Engine : public EngineBase {
   }
   template <int L, int CC>
   void pair_launch(const PairList<T>& li, int n, ColArgs a, const T* kv) {
-    constexpr int TPC = L / Plan<L>::E;
-    // one data region per group, and the twiddles' copy after them: up to the 160 KiB a gfx950
-    // workgroup can hold
+    constexpr int TPC = L / ColPlan<T, L>::E;
+    // one data region per group, then the copies of the twiddles and wavenumbers: up to the 160 KiB
+    // a gfx950 workgroup can hold
     constexpr long long PAIR_LDS_MAX = 160 * 1024;
     const long long region = (long long)L * CC * (long long)sizeof(C);
-    const long long twb = (long long)L * (long long)sizeof(C);
+    const long long copies = (long long)L * (long long)(sizeof(C) + sizeof(T));
     int G = std::max(1, 256 / (CC * TPC));
-    while (G > 1 && G * region + twb > PAIR_LDS_MAX) --G;
-    if (region + twb > PAIR_LDS_MAX) throw Error(GNSS_ERR_UNSUPPORTED, "late pass tile does not fit the LDS");
+    while (G > 1 && G * region + copies > LDS_MAX) --G;
+    if (region + copies > PAIR_LDS_MAX) throw Error(GNSS_ERR_UNSUPPORTED, "late pass tile does not fit the LDS");
     // the kernel takes the rows beyond the 2/3 rule's L / 3 for zeros without reading them
     if (a.in_keep != L / 3) throw Error(GNSS_ERR_STATE, "late pass input rows must be the kept ones");
     a.G = G;
-    const int threads = CC * TPC * G;
-    const size_t lds = (size_t)(G * region + twb);
     const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
-    const long long per_cu = std::max<long long>(1, std::min<long long>(160 * 1024 / (long long)lds, 2048 / threads));
-    const long long grid = std::min<long long>(blocks * n, per_cu * n_cu_);
-    hipLaunchKernelGGL((k_inv_late<T, L, CC>), dim3((unsigned)grid), dim3(threads), lds, s_, li, kv, tw_.at(L), a,
-                       (int)blocks, (int)(blocks * n));
+    hipLaunchKernelGGL((k_inv_late<T, L, CC>), dim3((unsigned)(blocks * n)), dim3(CC * TPC * G),
+                       (size_t)(G * region + copies), s_, li, kv, tw_.at(L), a, (int)blocks);
   }
 
   // x inverse passes of all work fields formed from the state (modes 2 and 3): one-input and

@@ -250,6 +250,19 @@ template <> struct Plan<384> { static constexpr int E = 12; using R = Radices<4,
 template <> struct Plan<512> { static constexpr int E = 8; using R = Radices<8, 8, 8>; };
 template <> struct Plan<1024> { static constexpr int E = 16; using R = Radices<16, 8, 8>; };
 
+// Plans of the strided passes' blocks.  A 512-point FP32 tile of 16 columns with eight elements per thread
+// is a block of 1024 threads, two of which leave 64 registers per lane; sixteen elements make it 512
+// threads with 128 registers, two blocks per CU either way.
+template <typename T, int L> struct ColPlan : Plan<L> {};
+template <> struct ColPlan<float, 512> { static constexpr int E = 16; using R = Radices<8, 8, 8>; };
+
+// Waves per SIMD of two blocks of a pass with C columns, the register budget to keep, when two fit the
+// LDS of a CU with their twiddles (and wavenumbers).
+template <typename T, int L, int C> __host__ __device__ constexpr int col_waves() {
+  const int threads = C * (L / ColPlan<T, L>::E) > 256 ? C * (L / ColPlan<T, L>::E) : 256;
+  return 2 * ((L * C + L) * 2 + L) * (int)sizeof(T) <= 160 * 1024 ? (2 * threads) / 256 : 1;
+}
+
 // Twiddle read: table tw[m] = exp(-2 pi i m / L); the inverse uses the conjugate.
 template <int SIGN, typename V> __device__ __forceinline__ V twid(const V* __restrict__ tw, int m) {
   V w = tw[m];

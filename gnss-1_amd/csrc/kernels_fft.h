@@ -111,18 +111,20 @@ template <typename T> struct FieldList {
   cx<T>* p[MAXW];
 };
 
-// One block per tile, field blockIdx.y.
+// One block per tile, field blockIdx.y.  The twiddles go through LDS, after the data regions (the first
+// stage uses none, and its exchange ends in a barrier, so the copy needs none of its own).
 template <typename T, int L, int SIGN, int C>
-__global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
+__global__ void __launch_bounds__(lb_threads(C * (L / ColPlan<T, L>::E)))
 k_col(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a) {
-  constexpr int E = Plan<L>::E;
+  using P = ColPlan<T, L>;
+  constexpr int E = P::E;
   constexpr int TPC = L / E;
   extern __shared__ unsigned char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int g = tid / (C * TPC);
+  const int g = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   const int chunk = blockIdx.x % a.nchunks;
   const int o = (blockIdx.x / a.nchunks) * a.G + g;
   bool active = o < a.nouter;
@@ -132,6 +134,8 @@ k_col(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a) {
   const TileRows in = tile_rows(a.sph, io, a.outer_n, chunk * C, a.in_keep);
   active = active && in.live;
   if (a.G == 1 && !active) return;
+  cx<T>* twl = lds + (long long)a.G * L * C;
+  for (int i = tid; i < L; i += blockDim.x) twl[i] = tw[i];
   const long long off = mo + (long long)io * a.ostride + (long long)chunk * C + c;
   const cx<T>* src = fl.in[blockIdx.y] + off;
   cx<T>* base = fl.p[blockIdx.y] + off;
@@ -142,7 +146,7 @@ k_col(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a) {
     if (active && row_kept(p, L, in.keep)) v[e] = ld_s(&src[(long long)p * a.estride]);
     else v[e] = mk<T>(0, 0);
   }
-  fft<T, L, SIGN>(v, lds, t, LdsCol{g * L * C + c, C}, tw);
+  fft<T, L, SIGN, LdsCol, P>(v, lds, t, LdsCol{g * L * C + c, C}, (const cx<T>*)twl);
   if (!active) return;
   const int out_keep = tile_rows(a.sph, io, a.outer_n, chunk * C, a.out_keep).keep;
 #pragma unroll
@@ -167,7 +171,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int g = tid / (C * TPC);
+  const int g = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   auto off_of = [&](int tile, TileRows& r, int box_keep) {
     const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;

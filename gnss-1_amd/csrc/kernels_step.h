@@ -622,7 +622,7 @@ k_xinv_prologue(Geom g, CPtrs<T> q, CPtrs<T> ws, const T* __restrict__ kxv, cons
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int gg = tid / (C * TPC);
+  const int gg = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   const int chunk = blockIdx.x % nchunks;
   const int o = (blockIdx.x / nchunks) * G + gg;
   const int nouter = 2 * g.keep_y + 1;
@@ -706,7 +706,7 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int g = tid / (C * TPC);
+  const int g = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   auto offset_of = [&](int tile, TileRows& r, int& iy, int& iz) {
     const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;
@@ -823,31 +823,29 @@ constexpr unsigned removed_slabs(int L, int TPC, int E) {
   return m;
 }
 
-// Persistent like k_xinv_op_pipe, over the entries of a whole pass: tile i is tile i % tpf of list entry
-// i / tpf, entries of one or two inputs and outputs together (the branches are uniform over the block), so
-// a pass is one launch with one tail.  Two outputs go through the radix stages one after the other in
-// one LDS region; the next tile's inputs are loaded once the last output is formed, ahead of its
-// transform.  Columns of removed modes are passed over and only rows inside the ellipsoid are loaded.
-// The twiddles are read from a copy in LDS, after the data regions: read from memory, each radix
-// stage would wait for every load in flight, the next tile's included.  An entry
-// may write its outputs over its own inputs (each tile is read before it is written, by the one
-// block that owns it, and both outputs are formed from registers); no entry may read a field
-// another entry writes.
+// One block per tile, over the entries of a whole pass: tile i is tile i % tpf of list entry i / tpf, entries
+// of one or two inputs and outputs together (the branches are uniform over the block), so a pass is one
+// launch.  Two outputs go through the radix stages one after the other in one LDS region, each from a
+// load of its own: the inputs stay in the L2, and a block keeps one set of values, which leaves room
+// for two blocks per CU whose transforms and memory phases overlap.  (As one persistent block per CU
+// that loaded the next tile ahead, its barriers put every wave into the same phase: 512^3 FP32 x 525 and
+// y 998 us per substage, now 431 and 959; FP64 992 -> 741 and 2030 -> 1800; 256^3 FP64 163 -> 119 and
+// 334 -> 276.)  Columns of removed modes end at once and only rows inside the ellipsoid are loaded.
+// The twiddles and the axis' wavenumbers are read from copies in LDS, after the data regions.  An entry
+// may write its outputs over its own inputs (the block that owns a tile writes output 0 last, over input
+// A, and output 1 only after reading B); no entry may read a field another entry writes.
 template <typename T, int L, int C>
-__global__ void __launch_bounds__(lb_threads(C * (L / Plan<L>::E)))
-k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ tw, ColArgs a, int tpf,
-           int ntiles) {
-  constexpr int E = Plan<L>::E;
+__global__ void __launch_bounds__(lb_threads(C * (L / ColPlan<T, L>::E)), (col_waves<T, L, C>()))
+k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ tw, ColArgs a, int tpf) {
+  using P = ColPlan<T, L>;
+  constexpr int E = P::E;
   constexpr int TPC = L / E;
   extern __shared__ unsigned char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int g = tid / (C * TPC);
-  // Element (row p = t + e TPC, column c) of a tile sits at tile_off(tile) + e TPC estride (the
-  // same for the whole group: with one group per block, wave-uniform) plus the lane's
-  // c + t estride, which the host keeps below 2^32 bytes.
+  const int g = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   auto tile_off = [&](int tile, TileRows& r) {
     const int lt = tile % tpf;
     const int chunk = lt % a.nchunks;
@@ -860,96 +858,54 @@ k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ t
     r.live = r.live && active;
     return mo + (long long)io * a.ostride + chunk * C;
   };
-  auto live_from = [&](int tile) {
-    if (a.G == 1 && a.sph.axis == 0) {
-      TileRows r;
-      for (; tile < ntiles; tile += gridDim.x) {
-        (void)tile_off(tile, r);
-        if (r.live) break;
-      }
-    }
-    return tile;
-  };
   const unsigned lane_b = (unsigned)(c + (long long)t * a.estride) * (unsigned)sizeof(cx<T>);
-  // the inputs hold the rows the 2/3 rule keeps (in_keep = L / 3, checked by the host): the slabs
-  // of removed rows are zeros known at compile time, neither loaded nor transformed
   constexpr unsigned ZS = removed_slabs(L, TPC, E);
-  cx<T> va[E], vb[E];
-  auto load_tile = [&](int tile) {
-    const int ent = tile / tpf;
-    TileRows r;
-    const long long off = tile_off(tile, r);
-    const cx<T>* __restrict__ A = li.A[ent];
+  const LdsCol idx{g * L * C + c, C};
+  cx<T>* twl = lds + (long long)a.G * L * C;
+  T* kl = reinterpret_cast<T*>(twl + L);
+  const int ent = blockIdx.x / tpf;
+  TileRows r;
+  const long long off = tile_off(blockIdx.x, r);
+  if (a.G == 1 && !r.live) return;
+  for (int i = tid; i < L; i += blockDim.x) {
+    twl[i] = tw[i];
+    kl[i] = kv[i];
+  }
+  auto load = [&](const cx<T>* __restrict__ src, cx<T>* v) {
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      va[e] = (!((ZS >> e) & 1u) && r.live && row_kept(t + e * TPC, L, r.keep))
-                  ? ld_at(A + off + (long long)e * TPC * a.estride, lane_b)
-                  : mk<T>(0, 0);
-    if (li.op[ent].nin == 2) {
-      const cx<T>* __restrict__ B = li.B[ent];
-#pragma unroll
-      for (int e = 0; e < E; ++e)
-        vb[e] = (!((ZS >> e) & 1u) && r.live && row_kept(t + e * TPC, L, r.keep))
-                    ? ld_at(B + off + (long long)e * TPC * a.estride, lane_b)
-                    : mk<T>(0, 0);
-    }
+      v[e] = (!((ZS >> e) & 1u) && r.live && row_kept(t + e * TPC, L, r.keep))
+                 ? ld_at(src + off + (long long)e * TPC * a.estride, lane_b)
+                 : mk<T>(0, 0);
   };
-  const LdsCol idx{g * L * C + c, C};
-  // the wavenumbers of this thread's rows, loaded once before the loop (see wait_vmem below)
-  T kr[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) kr[e] = kv[t + e * TPC];
-  int tile = live_from(blockIdx.x);
-  if (tile >= ntiles) return;
-  load_tile(tile);
-  cx<T>* twl = lds + (long long)a.G * L * C;
-  for (int i = tid; i < L; i += blockDim.x) twl[i] = tw[i];
-  // Nothing in flight when the loop starts: loads issued on paths that may skip some of them (the
-  // copy loop above, lane predicates) leave the compiler unable to count the loads in flight, and
-  // its first wait inside the loop would then be for every load, the next tile's included.
-  wait_vmem();
-  __syncthreads();
-  while (true) {
-    const int ent = tile / tpf;
-    const PairOp op = li.op[ent];
-    const int next = live_from(tile + gridDim.x);
-    const bool more = next < ntiles;
-    TileRows r;
-    const long long off = tile_off(tile, r);
+  // the second output first: the first may be written over the inputs
 #pragma unroll 1
-    for (int j = 0; j < op.nout; ++j) {
-      const T ra = (T)(j ? op.a[1] : op.a[0]), ba = (T)(j ? op.b[1] : op.b[0]);
-      const T rb = (T)(j ? op.c[1] : op.c[0]), db = (T)(j ? op.d[1] : op.d[0]);
-      cx<T> v[1][E];
+  for (int j = li.op[ent].nout - 1; j >= 0; --j) {
+    const PairOp* op = &li.op[ent];
+    const T ra = (T)(j ? op->a[1] : op->a[0]), ba = (T)(j ? op->b[1] : op->b[0]), rb = (T)(j ? op->c[1] : op->c[0]);
+    cx<T> v[1][E];
+    load(li.A[ent], v[0]);
+    __syncthreads();  // the copies are there, and the LDS of the last transform is free
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const T ka = ba * kl[t + e * TPC];
+      v[0][e] = mk<T>(ra * v[0][e].x - ka * v[0][e].y, ra * v[0][e].y + ka * v[0][e].x);
+    }
+    if (rb != (T)0) {
+      cx<T> vb[E];
+      load(li.B[ent], vb);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const T ka = ba * kr[e];
-        v[0][e] = mk<T>(ra * va[e].x - ka * va[e].y, ra * va[e].y + ka * va[e].x);
-      }
-      if (op.nin == 2) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const T kb = db * kr[e];
-          v[0][e].x += rb * vb[e].x - kb * vb[e].y;
-          v[0][e].y += rb * vb[e].y + kb * vb[e].x;
-        }
-      }
-      const bool last = j == op.nout - 1;
-      if (last && more) load_tile(next);
-      fft_batch<T, L, +1, LdsCol, Plan<L>, false, 1, L * C>(v, lds, t, idx, twl);
-      // one wait per tile, after its last transform and before its last stores: the counter
-      // covers loads and stores alike, so any wait with both in flight waits for all of them;
-      // here the next tile's loads have had a whole transform to arrive, where the compiler's
-      // own wait came after the stores and exposed their latency once per tile
-      if (last) wait_vmem();
-      if (r.live) {
-        cx<T>* __restrict__ dst = li.out[j][ent];
-#pragma unroll
-        for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[0][e]);
+        v[0][e].x += rb * vb[e].x;
+        v[0][e].y += rb * vb[e].y;
       }
     }
-    if (!more) break;
-    tile = next;
+    fft_batch<T, L, +1, LdsCol, P, false, 1, L * C>(v, lds, t, idx, twl);
+    if (r.live) {
+      cx<T>* __restrict__ dst = j ? li.out[1][ent] : li.out[0][ent];
+#pragma unroll
+      for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[0][e]);
+    }
   }
 }
 
@@ -983,7 +939,7 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
   const int tid = threadIdx.x;
   const int c = tid % C;
   const int t = (tid / C) % TPC;
-  const int gg = tid / (C * TPC);
+  const int gg = C * TPC >= 256 ? 0 : tid / (C * TPC);  // one group per block from 256 threads on
   const int chunk = blockIdx.x % nchunks;
   const int o = (blockIdx.x / nchunks) * G + gg;
   const int nouter = 2 * g.keep_y + 1;
