@@ -12,6 +12,7 @@
 #include <sstream>
 
 #include "engine.h"
+#include "host_link.h"
 #include "host_util.h"
 #include "kernels_fft.h"
 #include "kernels_mfma.h"
@@ -86,12 +87,13 @@ class Engine : public EngineBase {
     nsp_ = (long long)nx_ * ny_ * kzs_;
     nph_ = (long long)nx_ * ny_ * nz_;
     GNSS_HIP(hipStreamCreateWithFlags(&s_, hipStreamNonBlocking));
+    int dev = 0;
     {
-      int dev = 0;
       GNSS_HIP(hipGetDevice(&dev));
       GNSS_HIP(hipDeviceGetAttribute(&n_cu_, hipDeviceAttributeMultiprocessorCount, dev));
     }
     try {
+      link_.allocate(dev, std::max((size_t)nx_ * nzh_ * ny_ * sizeof(C), sizeof(T) * (size_t)nph_));
       allocate();
       qb_ = q_;
       dqb_ = dq_;
@@ -414,54 +416,75 @@ class Engine : public EngineBase {
     o->umax = sum[SPEC_NQ + 1];
   }
 
+  // Blocks of a kernel that moves a chunk over the bus: enough loads in flight for it, and no more.
+  static unsigned link_grid(long long n) { return (unsigned)std::min<long long>(cdiv(n, 256), 256); }
+  static void widen(const T* in, double* out, size_t n) {
+    if (sizeof(T) == sizeof(double)) memcpy(out, in, n * sizeof(double));
+    else
+      for (size_t i = 0; i < n; ++i) out[i] = (double)in[i];
+  }
+  static void narrow(const double* in, T* out, size_t n) {
+    if (sizeof(T) == sizeof(double)) memcpy(out, in, n * sizeof(double));
+    else
+      for (size_t i = 0; i < n; ++i) out[i] = (T)in[i];
+  }
+  void launch_done(const char* what, hipEvent_t ev) {
+    check_launch(what);
+    GNSS_HIP(hipEventRecord(ev, s_));
+  }
+
   void get_field(int f, int space, double* host) override {
     check_field(f);
     if (space == GNSS_PHYSICAL) {
-      std::vector<T> h(nph_);
-      GNSS_HIP(hipMemcpyAsync(h.data(), phys_[f], sizeof(T) * nph_, hipMemcpyDeviceToHost, s_));
-      sync();
-      for (long long i = 0; i < nph_; ++i) host[i] = (double)h[i];
+      const long long per = (long long)(link_.slot_bytes() / sizeof(T)) / 4 * 4;
+      link_.each((int)cdiv(nph_, per), [&](int c, void* mem, hipEvent_t ev) {
+        const long long i0 = c * per, n = std::min(per, nph_ - i0);
+        hipLaunchKernelGGL(k_real_copy<T>, dim3(link_grid(n / 4)), dim3(256), 0, s_, phys_[f] + i0, (T*)mem, n / 4);
+        launch_done("k_real_copy", ev);
+        GNSS_HIP(hipEventSynchronize(ev));
+        widen((const T*)mem, host + i0, (size_t)n);
+      });
       return;
     }
     if (space != GNSS_SPECTRAL) throw Error(GNSS_ERR_ARG, "bad space");
-    std::vector<C> h(nsp_);
-    GNSS_HIP(hipMemcpyAsync(h.data(), q_[f], sizeof(C) * nsp_, hipMemcpyDeviceToHost, s_));
-    sync();
-    for (int y = 0; y < ny_; ++y)
-      for (int x = 0; x < nx_; ++x) {
-        const C* src = h.data() + ((size_t)x * ny_ + y) * kzs_;
-        double* dst = host + 2 * ((size_t)y * nx_ + x) * nzh_;
-        for (int k = 0; k < nzh_; ++k) {
-          dst[2 * k] = (double)src[k].x;
-          dst[2 * k + 1] = (double)src[k].y;
-        }
-      }
+    const long long nrows = (long long)nx_ * ny_, per = rows_per_slot();
+    link_.each((int)cdiv(nrows, per), [&](int c, void* mem, hipEvent_t ev) {
+      const long long r0 = c * per, n = std::min(per, nrows - r0) * nzh_;
+      hipLaunchKernelGGL(k_spec_pack<T>, dim3(link_grid(n)), dim3(256), 0, s_, q_[f], (C*)mem, nx_, ny_, nzh_, kzs_, r0,
+                         n);
+      launch_done("k_spec_pack", ev);
+      GNSS_HIP(hipEventSynchronize(ev));
+      widen((const T*)mem, host + 2 * r0 * nzh_, (size_t)(2 * n));
+    });
   }
+  long long rows_per_slot() const { return (long long)(link_.slot_bytes() / sizeof(C)) / nzh_; }
 
   void set_field(int f, int space, const double* host) override {
     check_field(f);
     if (space == GNSS_PHYSICAL) {
-      std::vector<T> h(nph_);
-      for (long long i = 0; i < nph_; ++i) h[i] = (T)host[i];
-      GNSS_HIP(hipMemcpyAsync(phys_[f], h.data(), sizeof(T) * nph_, hipMemcpyHostToDevice, s_));
-      sync();
+      const long long per = (long long)(link_.slot_bytes() / sizeof(T)) / 4 * 4;
+      link_.each((int)cdiv(nph_, per), [&](int c, void* mem, hipEvent_t ev) {
+        const long long i0 = c * per, n = std::min(per, nph_ - i0);
+        narrow(host + i0, (T*)mem, (size_t)n);
+        hipLaunchKernelGGL(k_real_copy<T>, dim3(link_grid(n / 4)), dim3(256), 0, s_, (const T*)mem, phys_[f] + i0,
+                           n / 4);
+        launch_done("k_real_copy", ev);
+        GNSS_HIP(hipEventSynchronize(ev));
+      });
       return;
     }
     if (space != GNSS_SPECTRAL) throw Error(GNSS_ERR_ARG, "bad space");
     clean_ = false;
-    std::vector<C> h(nsp_);
-    memset((void*)h.data(), 0, sizeof(C) * nsp_);
-    for (int y = 0; y < ny_; ++y)
-      for (int x = 0; x < nx_; ++x) {
-        C* dst = h.data() + ((size_t)x * ny_ + y) * kzs_;
-        const double* src = host + 2 * ((size_t)y * nx_ + x) * nzh_;
-        for (int k = 0; k < nzh_; ++k) {
-          dst[k].x = (T)src[2 * k];
-          dst[k].y = (T)src[2 * k + 1];
-        }
-      }
-    GNSS_HIP(hipMemcpyAsync(q_[f], h.data(), sizeof(C) * nsp_, hipMemcpyHostToDevice, s_));
     GNSS_HIP(hipMemsetAsync(dq_[f], 0, sizeof(C) * nsp_, s_));
+    const long long nrows = (long long)nx_ * ny_, per = rows_per_slot();
+    link_.each((int)cdiv(nrows, per), [&](int c, void* mem, hipEvent_t ev) {
+      const long long r0 = c * per, rows = std::min(per, nrows - r0), n = rows * kzs_;
+      narrow(host + 2 * r0 * nzh_, (T*)mem, (size_t)(2 * rows * nzh_));
+      hipLaunchKernelGGL(k_spec_unpack<T>, dim3(link_grid(n)), dim3(256), 0, s_, (const C*)mem, q_[f], nx_, ny_, nzh_,
+                         kzs_, r0, n);
+      launch_done("k_spec_unpack", ev);
+      GNSS_HIP(hipEventSynchronize(ev));
+    });
     sync();
   }
 
@@ -1120,6 +1143,7 @@ class Engine : public EngineBase {
     allocs_.clear();
     if (scratch_) (void)hipFree(scratch_);
     scratch_ = nullptr;
+    link_.release();
     if (s_) (void)hipStreamDestroy(s_);
     s_ = nullptr;
   }
@@ -1926,6 +1950,7 @@ class Engine : public EngineBase {
   double t_ = 0;
   int64_t step_ = 0;
   KernelTimer timer_;
+  HostLink link_;
 };
 
 }  // namespace gnss

@@ -1106,6 +1106,34 @@ k_stats_reduce(const double* __restrict__ part, const double* __restrict__ spec,
   fin[t] = acc;
 }
 
+// Rows of a spectral field from row r0 on, in the ABI's order (row ky nx + kx, kz < nzh), to or from
+// host memory (pinned); unpacking also clears the kz padding.  Bound by the bus.
+template <typename T>
+__global__ void __launch_bounds__(256) k_spec_pack(const cx<T>* __restrict__ q, cx<T>* __restrict__ host, int nx, int ny,
+                                                   int nzh, int kzs, long long r0, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const long long r = i / nzh;
+    const int k = (int)(i - r * nzh), x = (int)((r0 + r) % nx), y = (int)((r0 + r) / nx);
+    host[i] = q[((long long)x * ny + y) * kzs + k];
+  }
+}
+template <typename T>
+__global__ void __launch_bounds__(256) k_spec_unpack(const cx<T>* __restrict__ host, cx<T>* __restrict__ q, int nx,
+                                                     int ny, int nzh, int kzs, long long r0, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const long long r = i / kzs;
+    const int k = (int)(i - r * kzs), x = (int)((r0 + r) % nx), y = (int)((r0 + r) / nx);
+    q[((long long)x * ny + y) * kzs + k] = k < nzh ? host[r * nzh + k] : mk<T>(0, 0);
+  }
+}
+// Contiguous values to or from host memory, four per thread and step (nz is a multiple of 8).
+template <typename T>
+__global__ void __launch_bounds__(256) k_real_copy(const T* __restrict__ in, T* __restrict__ out, long long n4) {
+  typedef T vec __attribute__((ext_vector_type(4)));
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long long)gridDim.x * blockDim.x)
+    reinterpret_cast<vec*>(out)[i] = reinterpret_cast<const vec*>(in)[i];
+}
+
 // Plain copy (bandwidth reference): block b copies the contiguous chunk [b chunk, (b + 1) chunk)
 // of 16-byte elements with four nontemporal loads in flight per thread before the stores.  Of the
 // copy forms measured on MI355X (grid-stride or chunked, 2-8 loads in flight, cached or
