@@ -57,10 +57,7 @@ class Engine : public EngineBase {
     if (colloid_ && !std::isfinite(p.alpha)) throw Error(GNSS_ERR_ARG, "alpha must be finite");
     F_ = 3 + S_;
     W_ = 6 + 3 * S_ + 2 * colloid_;
-    cx_ = col_chunk(nx_);
-    cy_ = col_chunk(ny_);
-    xc_ = cx_;
-    zf_ = 0;
+    default_tuning();
     load_tuning();  // may set kp, which fixes the row stride below
     // kz padding and the pruned kz limit use the widest column tile any variant may choose; kp
     // extra tiles of padding move the x pass's row stride (ny kzs elements) off large powers of two
@@ -977,8 +974,42 @@ class Engine : public EngineBase {
     return (long long)L * c * (long long)sizeof(C) <= LDS_MAX;
   }
 
+  // Pass variants by size and type, for grids without an entry in the table.  Measured over a middle
+  // substage (autotuner) of 16 grids from 24 x 192 x 16 to 512^3 in both precisions; us, FP32 / FP64:
+  //  * fields of a pass in one launch, one block per tile, the widest tiles (a tile half as wide costs 5 to
+  //    20 %): at 192^3 the late inverse mode takes 225 / 415, 247 / 456 with narrow tiles;
+  //  * x mode 4 or 5 (late derivatives): 192^3 225 against 254 (mode 2) and 491 FP64 (mode 1, the group-fused
+  //    prologue).  The forward x pass fused with the update (5) wins where its block is a power of two of
+  //    256 or 512 rows and there are tiles enough (512^3 3 329 / 6 708 against 3 418 / 6 936, 256^3 435 / 819
+  //    against 440 / 834); with 384 or 1024 rows its registers spill into the occupancy (384^3 1 805 / 3 491
+  //    against 1 760 / 3 422, 1024 x 128 x 96 516 against 494), and on small grids it waits longer than the
+  //    two launches it replaces (64^3 49 / 54 against 40 / 45).  The colloid has modes 0 to 3, the same two forms
+  //    being 2 and 3 (384 x 256 x 192: 1 133 / 2 038 in mode 2, 1 177 / 2 101 in 3, 1 216 / 2 174 in 1);
+  //  * fused z pass 9 (pairs of rows), but FP64 rows of 96 and of powers of two from 128 on variant 7 (33
+  //    against 39 us at 96^3, 38 against 42 at 128^3, 76 against 80 at 128 x 64 x 256, 2 191 against 2 396 at
+  //    512^3; 9 at 64^3: 10.2 against 11.8, at 192^3: 147 against 230, at 384^3: 1 284 against 2 017); the colloid
+  //    and rows of 1024 have 7 (384 x 256 x 192: 495 against 636 in variant 0);
+  //  * standalone z passes persistent in FP32 and on short FP64 rows (512^3 FP32 401 against 456, FP64 820
+  //    against 748).
+  void default_tuning() {
+    constexpr bool F32 = sizeof(T) == 4;
+    cx_ = col_chunk(nx_);
+    cy_ = col_chunk(ny_);
+    xc_ = cx_;
+    yc_ = 0;  // the late y passes' tile: as the x passes', unless those are narrower than need be
+    if (xc_ < (F32 ? 16 : 8) && ychunk_ok(F32 ? 16 : 8)) yc_ = F32 ? 16 : 8;
+    cb_ = 1;
+    cp_ = 0;
+    lp_ = 2;
+    zp_ = F32 || nz_ < 256 ? 1 : 0;
+    const bool fused_forward = (nx_ == 256 || nx_ == 512) && (double)nx_ * ny_ * nz_ >= 4.0e6;
+    xf_ = (fused_forward ? 1 : 0) + (colloid_ ? 2 : 4);
+    if (colloid_) zf_ = 7;
+    else zf_ = nz_ > 512 || (!F32 && (nz_ == 96 || (nz_ >= 128 && (nz_ & (nz_ - 1)) == 0))) ? 7 : 9;
+  }
+
   // Table of tuned choices: one line per key, "<key>": {"cx": C, "cy": C, "zf": V}.  Looked up in
-  // $GNSS_TUNING or tuning/gnss_tuning.json next to the library; absent entries keep defaults.
+  // $GNSS_TUNING or tuning/gnss_tuning.json next to the library; absent entries keep default_tuning's.
   void load_tuning() {
     std::string path;
     if (const char* e = getenv("GNSS_TUNING")) path = e;
