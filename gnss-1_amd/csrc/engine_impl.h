@@ -747,7 +747,7 @@ class Engine : public EngineBase {
     {
       int best = zf_;
       double best_ms = 1e30;
-      for (int v = 0; v <= 9; ++v) {
+      for (int v = 0; v <= 10; ++v) {
         if (!zvariant_ok(v)) continue;
         zf_ = v;
         const double ms = time_it([&] { z_fused(); });
@@ -881,7 +881,7 @@ class Engine : public EngineBase {
       {
         int best = zf_;
         double best_ms = 1e30;
-        for (int v = 0; v <= 9; ++v) {
+        for (int v = 0; v <= 10; ++v) {
           if (!zvariant_ok(v)) continue;
           zf_ = v;
           const double ms = time_it([&] { z_fused(); });
@@ -956,9 +956,9 @@ class Engine : public EngineBase {
 
  private:
   // fused z variants built: FP32 0-7 (8 is 7 in FP32), FP64 0, 3, 6, 7 and 8
-  // fused z variants built for this context (9, two rows per transform: no colloid, nz <= 512)
+  // fused z variants built for this context (two rows per transform: 9, with a colloid 10; nz <= 512)
   bool zvariant_ok(int v) const {
-    if (v == 9) return !colloid_ && nz_ <= 512;
+    if (v >= 9) return v == (colloid_ ? 10 : 9) && nz_ <= 512;
     return sizeof(T) == 4 ? (v >= 0 && v <= 7) : (v == 0 || v == 3 || (v >= 6 && v <= 8));
   }
   // column tiles the fused x kernels are built for: FP64 4 or 8, FP32 8 or 16
@@ -988,7 +988,7 @@ class Engine : public EngineBase {
   //  * fused z pass 9 (pairs of rows), but FP64 rows of 96 and of powers of two from 128 on variant 7 (33
   //    against 39 us at 96^3, 38 against 42 at 128^3, 76 against 80 at 128 x 64 x 256, 2 191 against 2 396 at
   //    512^3; 9 at 64^3: 10.2 against 11.8, at 192^3: 147 against 230, at 384^3: 1 284 against 2 017); the colloid
-  //    and rows of 1024 have 7 (384 x 256 x 192: 495 against 636 in variant 0);
+  //    has 10, its form of 9 (384 x 256 x 192 FP32: 277 us against 495 in 7 and 636 in 0), and rows of 1024 have 7;
   //  * standalone z passes persistent in FP32 and on short FP64 rows (512^3 FP32 401 against 456, FP64 820
   //    against 748).
   void default_tuning() {
@@ -1004,7 +1004,7 @@ class Engine : public EngineBase {
     zp_ = F32 || nz_ < 256 ? 1 : 0;
     const bool fused_forward = (nx_ == 256 || nx_ == 512) && (double)nx_ * ny_ * nz_ >= 4.0e6;
     xf_ = (fused_forward ? 1 : 0) + (colloid_ ? 2 : 4);
-    if (colloid_) zf_ = 7;
+    if (colloid_) zf_ = nz_ > 512 ? 7 : 10;
     else zf_ = nz_ > 512 || (!F32 && (nz_ == 96 || (nz_ >= 128 && (nz_ & (nz_ - 1)) == 0))) ? 7 : 9;
   }
 
@@ -1510,6 +1510,7 @@ class Engine : public EngineBase {
     }
     if constexpr (NZ <= 512) {
       if (zf_ == 9) return zfused_launch_v<NZ, 9>(a0, scale);
+      if (zf_ == 10) return zfused_launch_v<NZ, 10>(a0, scale);
     }
     zfused_launch_v<NZ, 0>(a0, scale);
   }
@@ -1520,8 +1521,8 @@ class Engine : public EngineBase {
     using P = typename FusedPlan<T, M, V>::type;
     constexpr int TPC = M / P::E;
     int G = std::max(1, 256 / TPC);
-    // LDS regions of one row: three fields of length M per radix stage, or (V = 9) PAIR_B rows of NZ
-    const long long row_lds = V == 9 ? (long long)PAIR_B * FusedPlan<T, M, V>::pad::stride(NZ) * (long long)sizeof(C)
+    // LDS regions of one row: three fields of length M per radix stage, or (V >= 9) PAIR_B rows of NZ
+    const long long row_lds = V >= 9 ? (long long)PAIR_B * FusedPlan<T, M, V>::pad::stride(NZ) * (long long)sizeof(C)
                                      : (long long)FUSED_B * FusedPlan<T, M, V>::pad::stride(M) * (long long)sizeof(C);
     while (G > 1 && G * row_lds > LDS_MAX) --G;
     ZFusedArgs<T> a = a0;

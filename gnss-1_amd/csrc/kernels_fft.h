@@ -660,6 +660,9 @@ template <typename T, int M> struct FusedPlan<T, M, 9> {
 };
 
 
+// V = 10: variant 9 with a colloid.
+template <typename T, int M> struct FusedPlan<T, M, 10> : FusedPlan<T, M, 9> {};
+
 // kz entries a substage's rows hold: kz <= nz/3 (the 2/3 rule), rounded up to the widest column tile
 // of the strided passes (16 complex in FP32, 8 in FP64); the engine's pruned kz limit.
 template <typename T> __host__ __device__ constexpr int zfused_lim(int nz) {
@@ -907,11 +910,13 @@ struct ZPair {
   }
 };
 
-// Fused z pass in pairs of rows (variant 9, no colloid): C2R of (u, v), (w, omega_x),
+// Fused z pass in pairs of rows (variants 9 and 10): C2R of (u, v), (w, omega_x),
 // (omega_y, omega_z), then per scalar (phi_x, phi_y), (phi_z, 0); R2C of the products paired in
 // order ((u x omega)_x, (u x omega)_y), ((u x omega)_z, u.grad phi_0), (u.grad phi_1, ...) ...
+// With a colloid (COL) its carrier Z = scalar 0 goes last of the plain scalars, after which the velocity
+// registers take the drift velocity u + alpha grad Z; then (c_x, c_y), (c_z, c) and (lap Z, 0).
 constexpr int PAIR_B = 2;  // packed rows per radix-stage batch (LDS regions per row of the block)
-template <typename T, int NZ, typename Pad, typename TW>
+template <typename T, int NZ, typename Pad, bool COL, typename TW>
 __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW& tw, T scale, cx<T>* lds, int t,
                                                 int g) {
   using Z = ZPair<T, NZ, Pad>;
@@ -962,20 +967,42 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
   Z::unpack_store(q[0], a.nl[0] + off, a.nl[1] + off, active, LIM, a.kzs, t, h);
   int pend_f = 2;  // product row waiting for a partner
   const typename Z::Raw zero{};
-  for (int s = 0; s < a.S; ++s) {
+  const int np = a.S - (COL ? 1 : 0);  // plain scalars
+  for (int i = 0; i < a.S; ++i) {
+    const bool col = COL && i == np;
+    const int s = !COL || col ? i : (i + 1 < np ? i + 1 : 0);
     const int w0 = 6 + 3 * s;
     H::load(a.ws[w0] + off, active, LIM, t, r[0]);
     H::load(a.ws[w0 + 1] + off, active, LIM, t, r[1]);
     if (a.late) H::template load_ikz<0, 1>(a.ws[w0 + 2] + off, a.ws[w0 + 2] + off, kzr, a.kz, active, LIM, t, r[2]);
     else H::load(a.ws[w0 + 2] + off, active, LIM, t, r[2]);
+    if (col) H::load(a.ws[6 + 3 * a.S] + off, active, LIM, t, r[3]);
     cx<T> zg[2][E];
     Z::pack(r[0], r[1], t, zg[0]);
-    Z::pack(r[2], zero, t, zg[1]);
+    if (col) Z::pack(r[2], r[3], t, zg[1]);
+    else Z::pack(r[2], zero, t, zg[1]);
     lds_sync<true>();
     fft_batch<T, N, +1, Pad, P, true, 2, RS>(zg, lds, t, idx, tw);
     T n[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) n[e] = za[0][e].x * zg[0][e].x + za[0][e].y * zg[0][e].y + w[e] * zg[1][e].x;
+    if constexpr (COL) {
+      if (!col && s == 0) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          za[0][e].x += a.alpha * zg[0][e].x;
+          za[0][e].y += a.alpha * zg[0][e].y;
+          w[e] += a.alpha * zg[1][e].x;
+        }
+      } else if (col) {
+        H::load(a.ws[7 + 3 * a.S] + off, active, LIM, t, r[0]);
+        Z::pack(r[0], zero, t, zb[0]);
+        lds_sync<true>();
+        fft_batch<T, N, +1, Pad, P, true, 1, RS>(zb, lds, t, idx, tw);
+#pragma unroll
+        for (int e = 0; e < E; ++e) n[e] += a.alpha * zb[0][e].x * zg[1][e].y;
+      }
+    }
     if (pend_f >= 0) {
 #pragma unroll
       for (int e = 0; e < E; ++e) q[0][e] = mk<T>(pend[e], n[e]);
@@ -1008,10 +1035,10 @@ k_zfused(ZFusedArgs<T> a, const cx<T>* __restrict__ twM, const cx<T>* __restrict
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int t = threadIdx.x % Z::TPC;
   const int g = Z::TPC == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : threadIdx.x / Z::TPC;
-  if constexpr (V == 9) {
+  if constexpr (V == 9 || V == 10) {
     TwRegs<T, NZ, Plan<NZ>> tw;
     tw.load(twN, t);
-    zfused_pair_row<T, NZ, typename FP::pad>(a, tw, scale, lds, t, g);
+    zfused_pair_row<T, NZ, typename FP::pad, V == 10>(a, tw, scale, lds, t, g);
   } else if constexpr (FP::regtw) {
     typename Z::Tw tw;
     tw.load(twM, twN, t);
