@@ -985,10 +985,11 @@ class Engine : public EngineBase {
   //    against 1 760 / 3 422, 1024 x 128 x 96 516 against 494), and on small grids it waits longer than the
   //    two launches it replaces (64^3 49 / 54 against 40 / 45).  The colloid has modes 0 to 3, the same two forms
   //    being 2 and 3 (384 x 256 x 192: 1 133 / 2 038 in mode 2, 1 177 / 2 101 in 3, 1 216 / 2 174 in 1);
-  //  * fused z pass 9 (pairs of rows), but FP64 rows of 96 and of powers of two from 128 on variant 7 (33
-  //    against 39 us at 96^3, 38 against 42 at 128^3, 76 against 80 at 128 x 64 x 256, 2 191 against 2 396 at
-  //    512^3; 9 at 64^3: 10.2 against 11.8, at 192^3: 147 against 230, at 384^3: 1 284 against 2 017); the colloid
-  //    has 10, its form of 9 (384 x 256 x 192 FP32: 277 us against 495 in 7 and 636 in 0), and rows of 1024 have 7;
+  //  * fused z pass: FP64 rows of powers of two from 64 on variant 7, whose exchanges are lane swaps from 128 on
+  //    (128^2 rows of 64: 24 us against 27 in variant 9, of 128: 41 against 50, of 256: 76 against 88, of 512: 144
+  //    against 167); everything else in pairs of rows, 9 or with a colloid 10 (128^2 rows of 96: FP64 62 against
+  //    79, FP32 26 against 51; FP32 rows of 512: 76 against 87; with a colloid FP32 rows of 192 53 against 99, FP64
+  //    114 against 163, but FP64 rows of 256 180 against 101); rows of 1024 have 7 only;
   //  * standalone z passes persistent in FP32 and on short FP64 rows (512^3 FP32 401 against 456, FP64 820
   //    against 748).
   void default_tuning() {
@@ -1004,8 +1005,8 @@ class Engine : public EngineBase {
     zp_ = F32 || nz_ < 256 ? 1 : 0;
     const bool fused_forward = (nx_ == 256 || nx_ == 512) && (double)nx_ * ny_ * nz_ >= 4.0e6;
     xf_ = (fused_forward ? 1 : 0) + (colloid_ ? 2 : 4);
-    if (colloid_) zf_ = nz_ > 512 ? 7 : 10;
-    else zf_ = nz_ > 512 || (!F32 && (nz_ == 96 || (nz_ >= 128 && (nz_ & (nz_ - 1)) == 0))) ? 7 : 9;
+    const bool pow2 = (nz_ & (nz_ - 1)) == 0;
+    zf_ = nz_ > 512 || (!F32 && pow2 && nz_ >= 64) ? 7 : (colloid_ ? 10 : 9);
   }
 
   // Table of tuned choices: one line per key, "<key>": {"cx": C, "cy": C, "zf": V}.  Looked up in

@@ -297,7 +297,9 @@ template <typename T, int L, typename P> struct TwRegs {
   static constexpr int total = off(L);
   cx<T> w[total > 0 ? total : 1];
 
-  __device__ __forceinline__ void load(const cx<T>* __restrict__ tw, int t) {
+  // t4: the thread's position in the stage of span 4, where that differs (see LaneFft)
+  __device__ __forceinline__ void load(const cx<T>* __restrict__ tw, int t) { load(tw, t, t); }
+  __device__ __forceinline__ void load(const cx<T>* __restrict__ tw, int t, int t4) {
     constexpr int TPC = L / E;
     int s = 1, o = 0;
 #pragma unroll
@@ -306,7 +308,7 @@ template <typename T, int L, typename P> struct TwRegs {
       if (s > 1) {
 #pragma unroll
         for (int bt = 0; bt < NB; ++bt) {
-          const int k = (t + bt * TPC) % s;
+          const int k = ((s == 4 ? t4 : t) + bt * TPC) % s;
 #pragma unroll
           for (int r = 1; r < R; ++r) w[o + bt * (R - 1) + r - 1] = tw[r * k * (L / (s * R))];
         }
@@ -449,6 +451,109 @@ template <typename T, int L, int SIGN, typename Idx, typename P, bool WAVE, int 
 __device__ __forceinline__ void fft_batch(cx<T> (*v)[P::E], cx<T>* lds, int t, const Idx& idx, const TW& tw) {
   static_assert(!WAVE || (L / P::E) <= 64, "a wave-synchronised transform must fit one wavefront");
   FftL<T, L, SIGN, Idx, P, WAVE, B, BSTRIDE, typename P::R>::run(v, lds, t, idx, tw);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Transforms of one wavefront whose exchanges go through lane swaps.
+//
+// An exchange between two radix-4 stages moves the register index q of a value into its thread's index
+// and the thread index' top two bits into the register index.  If those two bits are lane bits 5 and
+// 4, that is a transposition of registers with lane halves and lane rows: one permlane32/16 swap per pair
+// of registers instead of an LDS write and read.  Which lane then holds which thread index has changed
+// (q sits in lane bits 5 and 4 but in index bits log2(span) on), so the next exchange cannot do the same:
+// it goes through LDS and puts every index back in its place.
+// ---------------------------------------------------------------------------------------------
+// Lanes of a wave with 64 / TPC transforms of TPC threads: contiguous, or with the top two bits of the
+// thread index in lane bits 5 and 4 and the transform's number between them and the low bits.
+template <int TPC> struct LaneRuns {
+  __device__ __forceinline__ static int thread(int lane) { return lane & (TPC - 1); }
+  __device__ __forceinline__ static int row(int lane) { return lane / TPC; }
+  __device__ __forceinline__ static int lane(int row, int t) { return row * TPC + t; }
+};
+template <int TPC> struct LaneTop {
+  static constexpr int LOW = TPC / 4;
+  __device__ __forceinline__ static int thread(int lane) { return (lane >> 4) * LOW + (lane & (LOW - 1)); }
+  __device__ __forceinline__ static int row(int lane) { return (lane & 15) / LOW; }
+  __device__ __forceinline__ static int lane(int row, int t) { return ((t / LOW) << 4) + row * LOW + (t & (LOW - 1)); }
+  // the thread index a lane holds after the exchange of span 1: its low bits moved up, q in the lowest
+  __device__ __forceinline__ static int swapped(int lane) { return (lane & (LOW - 1)) * 4 + (lane >> 4); }
+};
+
+// Lanes 32-63 of a with lanes 0-31 of b (ROW: lanes 16-31 and 48-63 of a with 0-15 and 32-47 of b).
+template <bool ROW> __device__ __forceinline__ void lane_swap(double& a, double& b) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  u2 x, y;
+  __builtin_memcpy(&x, &a, 8);
+  __builtin_memcpy(&y, &b, 8);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = ROW ? __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false)
+                       : __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+    x[i] = r[0];
+    y[i] = r[1];
+  }
+  __builtin_memcpy(&a, &x, 8);
+  __builtin_memcpy(&b, &y, 8);
+}
+template <bool ROW, typename V> __device__ __forceinline__ void lane_swap_c(V& a, V& b) {
+  lane_swap<ROW>(a.x, b.x);
+  lane_swap<ROW>(a.y, b.y);
+}
+// register index (q1 q0) <-> lane bits (5, 4)
+template <typename V> __device__ __forceinline__ void lane_swap4(V* v) {
+  lane_swap_c<false>(v[0], v[2]);
+  lane_swap_c<false>(v[1], v[3]);
+  lane_swap_c<true>(v[0], v[1]);
+  lane_swap_c<true>(v[2], v[3]);
+}
+
+// B transforms of length M = 64, 128 or 256 with four values per thread, lanes as LaneTop<M / 4> (plan
+// PlanLow<M>, stages 4 4 4 [2 or 4], twiddles from a TwRegs loaded with LaneTop's swapped index for span 4):
+// the exchanges of span 1 and 16 are lane swaps, that of span 4 goes through LDS.
+template <typename T, int M, int SIGN, typename Idx, int B, int BSTRIDE, typename TW>
+__device__ __forceinline__ void fft_lanes(cx<T> (*v)[4], cx<T>* lds, int t, const Idx& idx, const TW& tw) {
+  static_assert(M == 64 || M == 128 || M == 256, "lane-swap plans");
+  using V = cx<T>;
+  const int ts = LaneTop<M / 4>::swapped(threadIdx.x & 63);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    Dft<4, SIGN, V>::run(v[b]);
+    lane_swap4(v[b]);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) v[b][r] = cmul(v[b][r], stage_tw<SIGN, M, 4, 4, V>(tw, 0, 0, r));
+    Dft<4, SIGN, V>::run(v[b]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) lds[idx((ts / 4) * 16 + (ts & 3) + 4 * q) + b * BSTRIDE] = v[b][q];
+  }
+  lds_sync<true>();
+#pragma unroll
+  for (int b = 0; b < B; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[b][e] = lds[idx(t + e * (M / 4)) + b * BSTRIDE];
+  lds_sync<true>();
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+#pragma unroll
+    for (int r = 1; r < 4; ++r) v[b][r] = cmul(v[b][r], stage_tw<SIGN, M, 16, 4, V>(tw, 0, 0, r));
+    Dft<4, SIGN, V>::run(v[b]);
+    if constexpr (M == 256) {
+      lane_swap4(v[b]);
+#pragma unroll
+      for (int r = 1; r < 4; ++r) v[b][r] = cmul(v[b][r], stage_tw<SIGN, M, 64, 4, V>(tw, 0, 0, r));
+      Dft<4, SIGN, V>::run(v[b]);
+    } else if constexpr (M == 128) {
+      // the top register index is the old top thread bit, the lower one q1; q0 takes that thread bit
+      lane_swap_c<false>(v[b][0], v[b][1]);
+      lane_swap_c<false>(v[b][2], v[b][3]);
+      V a[4] = {v[b][0], v[b][2], v[b][1], v[b][3]};
+#pragma unroll
+      for (int bt = 0; bt < 2; ++bt) {
+        const V w = cmul(a[bt + 2], stage_tw<SIGN, M, 64, 2, V>(tw, 0, bt, 1));
+        v[b][bt] = cadd(a[bt], w);
+        v[b][bt + 2] = csub(a[bt], w);
+      }
+    }
+  }
 }
 
 // Signed mode index of storage index i along an axis of length n.

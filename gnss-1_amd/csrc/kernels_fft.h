@@ -251,13 +251,21 @@ __host__ __device__ constexpr int zrow_stride(int M) { return M + 2 + (M >> 4); 
 // values is packed as M = NZ/2 complex pairs (z = 2n, 2n+1); the half-length transform is
 // unpacked with exp(-2 pi i k / NZ) (R2C) or packed the same way before it (C2R).  TPC divides
 // 64, so a row never straddles wavefronts and all row-local LDS traffic is wave-synchronised.
-template <typename T, int NZ, typename P, typename Pad = LdsRow>
+// LANES: the transforms' exchanges are lane swaps where they can be (fft_lanes), lanes as LaneTop.
+template <typename T, int NZ, typename P, typename Pad = LdsRow, bool LANES = false>
 struct ZRow {
   static constexpr int M = NZ / 2;
   static constexpr int E = P::E;
   static constexpr int TPC = M / E;
   static constexpr int RS = Pad::stride(M);
   static_assert(64 % TPC == 0, "a z row must lie inside one wavefront");
+  using Lanes = typename std::conditional<LANES, LaneTop<LANES ? TPC : 4>, LaneRuns<TPC>>::type;
+  // the transforms of B rows
+  template <int SIGN, int B, typename TM>
+  __device__ __forceinline__ static void rows_fft(cx<T> (*v)[E], cx<T>* lds, const Pad& idx, int t, const TM& tw) {
+    if constexpr (LANES) fft_lanes<T, M, SIGN, Pad, B, RS>(v, lds, t, idx, tw);
+    else fft_batch<T, M, SIGN, Pad, P, true, B, RS>(v, lds, t, idx, tw);
+  }
 
   // Registers of one spectral row as loaded from HBM (entries k >= lim read as 0); thread 0 also
   // holds Re X[M] in nyq (a register of its own: loaded into half of x[0], it would have to wait
@@ -319,7 +327,8 @@ struct ZRow {
     TwRegs<T, M, P> m;
     cx<T> n[E / 2];
     __device__ __forceinline__ void load(const cx<T>* __restrict__ twM, const cx<T>* __restrict__ twN, int t) {
-      m.load(twM, t);
+      if constexpr (LANES) m.load(twM, t, Lanes::swapped(threadIdx.x & 63));
+      else m.load(twM, t);
 #pragma unroll
       for (int e = 0; e < E / 2; ++e) n[e] = twN[t + e * TPC];
     }
@@ -336,8 +345,14 @@ struct ZRow {
   __device__ __forceinline__ static cx<T> mirror(const cx<T>& x, int t) {
     const int src = (TPC - t) & (TPC - 1);
     cx<T> r;
-    r.x = __shfl(x.x, src, TPC);
-    r.y = __shfl(x.y, src, TPC);
+    if constexpr (LANES) {
+      const int lane = Lanes::lane(Lanes::row(threadIdx.x & 63), src);
+      r.x = __shfl(x.x, lane, 64);
+      r.y = __shfl(x.y, lane, 64);
+    } else {
+      r.x = __shfl(x.x, src, TPC);
+      r.y = __shfl(x.y, src, TPC);
+    }
     return r;
   }
 
@@ -380,7 +395,7 @@ struct ZRow {
       }
     }
     lds_sync<true>();
-    fft_batch<T, M, +1, Pad, P, true, B, RS>(v, lds, t, idx, mtw(twM, twN));
+    rows_fft<+1, B>(v, lds, idx, t, mtw(twM, twN));
     if constexpr (SCALE) {
 #pragma unroll
       for (int b = 0; b < B; ++b)
@@ -397,7 +412,7 @@ struct ZRow {
                                              int kzs, cx<T>* lds, const Pad& idx, int t, const TM& twM,
                                              const TN& twN, T h = (T)0.5, bool drain = false) {
     lds_sync<true>();
-    fft_batch<T, M, -1, Pad, P, true, B, RS>(v, lds, t, idx, mtw(twM, twN));
+    rows_fft<-1, B>(v, lds, idx, t, mtw(twM, twN));
     // drain: wait for every memory operation in flight before the stores (a pipelined caller's
     // next rows, loaded before the transform; see wait_vmem)
     if (drain) wait_vmem();
@@ -638,6 +653,13 @@ template <typename T, int M> struct FusedPlan<T, M, 6> : FusedPlan<T, M, 3> {
 template <typename T, int M> struct FusedPlan<T, M, 7> : FusedPlan<T, M, 6> {
   static constexpr bool defer = true;
 };
+// FP64 rows of 128, 256 and 512 in variant 7 exchange through lane swaps where they can: their pass was bound by
+// the LDS (at 512^3 4.0 k LDS cycles per row of 2.2 k vector instructions, a third of them bank conflicts), and
+// two of three exchanges leave it (rows of 256 98 -> 76 us, of 512 193 -> 144 at 128^2 rows and one scalar; 512^3
+// 2.39 -> 2.18 ms).  The FP32 forms are bound by vector instructions, which the swaps are too.
+template <typename T, int M, int V> constexpr bool lane_rows() {
+  return sizeof(T) == 8 && V == 7 && (M == 64 || M == 128 || M == 256);
+}
 template <typename T, int M> struct FusedPlan<T, M, 8> : FusedPlan<T, M, 7> {
   using pad = typename std::conditional<sizeof(T) == 4, LdsRowP<5, 5>, LdsRowP<3, 2>>::type;
 };
@@ -709,7 +731,7 @@ template <typename T, int NZ, int V, typename TM, typename TN>
 __device__ __forceinline__ void zfused_row(const ZFusedArgs<T>& a, const TM& twM, const TN& twN, T scale,
                                            cx<T>* lds, int t, int g) {
   using FP = FusedPlan<T, NZ / 2, V>;
-  using Z = ZRow<T, NZ, typename FP::type, typename FP::pad>;
+  using Z = ZRow<T, NZ, typename FP::type, typename FP::pad, lane_rows<T, NZ / 2, V>()>;
   constexpr int E = Z::E;
   constexpr bool PREFETCH = FP::prefetch;
   // Variants with `defer`: the inverse transforms skip their 1/N; every product below is quadratic
@@ -1030,11 +1052,13 @@ __global__ void __launch_bounds__(lb_threads((NZ / 2) / FusedPlan<T, NZ / 2, V>:
                                   (FusedPlan<T, NZ / 2, V>::min_waves))
 k_zfused(ZFusedArgs<T> a, const cx<T>* __restrict__ twM, const cx<T>* __restrict__ twN, T scale) {
   using FP = FusedPlan<T, NZ / 2, V>;
-  using Z = ZRow<T, NZ, typename FP::type, typename FP::pad>;
+  using Z = ZRow<T, NZ, typename FP::type, typename FP::pad, lane_rows<T, NZ / 2, V>()>;
   extern __shared__ unsigned char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-  const int t = threadIdx.x % Z::TPC;
-  const int g = Z::TPC == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : threadIdx.x / Z::TPC;
+  const int lane = threadIdx.x & 63;
+  const int t = Z::Lanes::thread(lane);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int g = wave * (64 / Z::TPC) + Z::Lanes::row(lane);
   if constexpr (V == 9 || V == 10) {
     TwRegs<T, NZ, Plan<NZ>> tw;
     tw.load(twN, t);
