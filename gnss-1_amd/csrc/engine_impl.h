@@ -1522,8 +1522,8 @@ class Engine : public EngineBase {
     using P = typename FusedPlan<T, M, V>::type;
     constexpr int TPC = M / P::E;
     int G = std::max(1, 256 / TPC);
-    // LDS regions of one row: three fields of length M per radix stage, or (V >= 9) PAIR_B rows of NZ
-    const long long row_lds = V >= 9 ? (long long)PAIR_B * FusedPlan<T, M, V>::pad::stride(NZ) * (long long)sizeof(C)
+    // LDS regions of one row: three fields of length M per radix stage, or (V >= 9) pair_b rows of NZ
+    const long long row_lds = V >= 9 ? (long long)pair_b<T, NZ>() * FusedPlan<T, M, V>::pad::stride(NZ) * (long long)sizeof(C)
                                      : (long long)FUSED_B * FusedPlan<T, M, V>::pad::stride(M) * (long long)sizeof(C);
     while (G > 1 && G * row_lds > LDS_MAX) --G;
     ZFusedArgs<T> a = a0;

@@ -937,7 +937,12 @@ struct ZPair {
 // order ((u x omega)_x, (u x omega)_y), ((u x omega)_z, u.grad phi_0), (u.grad phi_1, ...) ...
 // With a colloid (COL) its carrier Z = scalar 0 goes last of the plain scalars, after which the velocity
 // registers take the drift velocity u + alpha grad Z; then (c_x, c_y), (c_z, c) and (lap Z, 0).
-constexpr int PAIR_B = 2;  // packed rows per radix-stage batch (LDS regions per row of the block)
+// Packed rows per radix-stage batch (LDS regions per row of the block).  Two share each exchange's latency,
+// but rows of 12 values per thread then fill the LDS with two blocks of a CU, eight waves, where FP32's
+// registers allow twelve: those go one by one (192^2 rows of 96: 58 -> 52 us, of 192: 85 -> 75, 384^3: 690 ->
+// 578).  FP64's registers allow four waves; two rows at a time are better there (rows of 192: 173 against 187
+// us, 384^3: 1 363 against 1 583) but for the shortest (rows of 96: 137 against 106).
+template <typename T, int NZ> constexpr int pair_b() { return Plan<NZ>::E == 12 && (sizeof(T) == 4 || NZ <= 96) ? 1 : 2; }
 template <typename T, int NZ, typename Pad, bool COL, typename TW>
 __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW& tw, T scale, cx<T>* lds, int t,
                                                 int g) {
@@ -950,7 +955,8 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
   const long long row = (long long)blockIdx.x * a.G + g;
   const bool active = row < a.nrows;
   const long long off = (active ? row : 0) * a.kzs;
-  const Pad idx{g * RS * PAIR_B};
+  constexpr int PB = pair_b<T, NZ>();
+  const Pad idx{g * RS * PB};
   T kzr[HE];
 #pragma unroll
   for (int e = 0; e < HE; ++e) kzr[e] = (a.late && t + e * Z::TPC < LIM) ? a.kz[t + e * Z::TPC] : (T)0;
@@ -965,7 +971,11 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
   Z::pack(r[0], r[1], t, za[0]);
   Z::pack(r[2], r[3], t, za[1]);
   lds_sync<true>();
-  fft_batch<T, N, +1, Pad, P, true, 2, RS>(za, lds, t, idx, tw);
+  fft_batch<T, N, +1, Pad, P, true, PB, RS>(za, lds, t, idx, tw);
+  if constexpr (PB == 1) {
+    lds_sync<true>();
+    fft_batch<T, N, +1, Pad, P, true, 1, RS>(za + 1, lds, t, idx, tw);
+  }
   if (a.late) H::template load_ikz<-1, 1>(a.ws[4] + off, a.ws[0] + off, kzr, a.kz, active, LIM, t, r[0]);
   else H::load(a.ws[4] + off, active, LIM, t, r[0]);
   H::load(a.ws[5] + off, active, LIM, t, r[1]);
@@ -1004,7 +1014,11 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
     if (col) Z::pack(r[2], r[3], t, zg[1]);
     else Z::pack(r[2], zero, t, zg[1]);
     lds_sync<true>();
-    fft_batch<T, N, +1, Pad, P, true, 2, RS>(zg, lds, t, idx, tw);
+    fft_batch<T, N, +1, Pad, P, true, PB, RS>(zg, lds, t, idx, tw);
+    if constexpr (PB == 1) {
+      lds_sync<true>();
+      fft_batch<T, N, +1, Pad, P, true, 1, RS>(zg + 1, lds, t, idx, tw);
+    }
     T n[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) n[e] = za[0][e].x * zg[0][e].x + za[0][e].y * zg[0][e].y + w[e] * zg[1][e].x;
