@@ -91,6 +91,7 @@ class Engine : public EngineBase {
     }
     try {
       link_.allocate(dev, std::max((size_t)nx_ * nzh_ * ny_ * sizeof(C), sizeof(T) * (size_t)nph_));
+      flag_ = link_.flag();
       allocate();
       qb_ = q_;
       dqb_ = dq_;
@@ -272,17 +273,15 @@ class Engine : public EngineBase {
 
   // NaN/Inf watchdog on the kz = 0 column of every field.
   void check_finite() override {
-    GNSS_HIP(hipMemsetAsync(d_flag_, 0, sizeof(int), s_));
+    *flag_ = 0;  // nothing that writes it is in flight: every check ends in a synchronisation
     for (int m = 0; m < nb_; ++m) {
       if (nb_ > 1) select_member(m);
-      hipLaunchKernelGGL(k_finite<T>, dim3(cdiv((long long)nx_ * ny_, 256)), dim3(256), 0, s_, g_,
-                         ptrs(q_), F_, d_flag_);
+      hipLaunchKernelGGL(k_finite<T>, dim3(cdiv((long long)nx_ * ny_, 256), F_), dim3(256), 0, s_, g_, ptrs(q_), flag_);
       check_launch("k_finite");
     }
     if (nb_ > 1) select_member(0);
-    int flag = 0;
-    GNSS_HIP(hipMemcpyAsync(&flag, d_flag_, sizeof(int), hipMemcpyDeviceToHost, s_));
     sync();
+    const int flag = *(volatile int*)flag_;
     if (flag) throw Error(GNSS_ERR_NUMERIC, "non-finite value in the state after step " + std::to_string(step_));
   }
 
@@ -622,8 +621,11 @@ class Engine : public EngineBase {
     } else {
       CPtrs<T> w{};
       for (int c = 0; c < 3; ++c) w.p[c] = ws_[c];
-      hipLaunchKernelGGL(k_vorticity<T>, dim3((unsigned)cdiv(nsp_, 256)), dim3(256), 0, s_, g_, ptrs(q_), w, tkx_,
-                         tky_, tkz_, nsp_);
+      Box b = kept_box();
+      if (!clean_) b = Box{nx_, ny_, kzs_, -1, -1};
+      const long long nm = (long long)b.bx * b.by * b.bz;
+      hipLaunchKernelGGL(k_vorticity<T>, dim3((unsigned)cdiv(nm, 256)), dim3(256), 0, s_, g_, b, ptrs(q_), w, tkx_,
+                         tky_, tkz_, nm);
       T* om[3];
       for (int c = 0; c < 3; ++c) om[c] = reinterpret_cast<T*>(ws_[3 + c]);
       inv3d(ws_.data(), ws_.data(), om, 3, clean_);
@@ -652,13 +654,15 @@ class Engine : public EngineBase {
     const T* a = diag_field(field);
     const double dx = p_.lx / nx_, dy = p_.ly / ny_, dz = p_.lz / nz_;
     timed("k_surface_area", (double)nph_ * sizeof(T), [&] {
-      hipLaunchKernelGGL(k_surface_area<T>, dim3(nx_), dim3(STAT_THREADS), 0, s_, g_, a, iso, dx, dy, dz, d_part_);
+      hipLaunchKernelGGL(k_surface_area<T>, dim3(nx_, AREA_SPLIT), dim3(AREA_THREADS), 0, s_, g_, a, iso, dx, dy, dz,
+                         d_part_);
     });
-    std::vector<double> part(nx_);
-    GNSS_HIP(hipMemcpyAsync(part.data(), d_part_, sizeof(double) * nx_, hipMemcpyDeviceToHost, s_));
+    static_assert(AREA_SPLIT <= SPEC_NQ, "the partial areas use the spectral sums' buffer");
+    std::vector<double> part((size_t)nx_ * AREA_SPLIT);
+    GNSS_HIP(hipMemcpyAsync(part.data(), d_part_, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s_));
     sync();
     double sum = 0.0;
-    for (int x = 0; x < nx_; ++x) sum += part[x];
+    for (double v : part) sum += v;
     return sum * dx * dy * dz;
   }
 
@@ -1116,7 +1120,6 @@ class Engine : public EngineBase {
       dalloc(phys_[f], sizeof(T) * nph_);
     }
     for (int w = 0; w < W_; ++w) dalloc(ws_[w], sizeof(C) * nst);
-    for (void* v : allocs_) GNSS_HIP(hipMemsetAsync(v, 0, 1, s_));
     for (int f = 0; f < F_; ++f) {
       GNSS_HIP(hipMemsetAsync(q_[f], 0, sizeof(C) * nst, s_));
       GNSS_HIP(hipMemsetAsync(dq_[f], 0, sizeof(C) * nst, s_));
@@ -1139,7 +1142,6 @@ class Engine : public EngineBase {
     dalloc(d_prof_, sizeof(double) * (size_t)(7 + 3 * S_) * ny_);
     dalloc(d_cmax_, sizeof(double) * 2 * ny_);
     dalloc(d_fin_, sizeof(double) * (SPEC_NQ + 2 + (size_t)(1 + S_) * nb));
-    dalloc(d_flag_, sizeof(int));
     // twiddle tables for every length the passes use
     for (int L : {nx_, ny_, nz_, nz_ / 2}) {
       if (tw_.count(L)) continue;
@@ -1625,10 +1627,24 @@ class Engine : public EngineBase {
       l.op[n] = op;
       ++n;
     };
+    // Small grids take a field and its x derivative in blocks of their own (the passes' outputs are not their
+    // inputs): the launch then lasts one transform instead of two.
+    const int CC = pair_chunk(), CY = yc_ ? yc_ : CC;
+    const long long xtiles = (long long)(kz_lim_ / CC) * (2 * g_.keep_y + 1) * bm_ * (3 + S_);
+    const bool apart = xtiles * (CC * nx_ / elems_per_thread(nx_)) <= (long long)n_cu_ * 1024;
+    const PairOp deriv{1, 1, {0, 0}, {1, 0}, {0, 0}, {0, 0}};       // out0 = i k A
+    auto put_d = [&](const C* A, C* o0, C* o1) {
+      if (apart) {
+        put(lx, nxe, A, nullptr, o0, nullptr, copy);
+        put(lx, nxe, A, nullptr, o1, nullptr, deriv);
+      } else {
+        put(lx, nxe, A, nullptr, o0, o1, copy_d);
+      }
+    };
     put(lx, nxe, q_[0], nullptr, ws_[0], nullptr, copy);
-    put(lx, nxe, q_[1], nullptr, ws_[1], ws_[5], copy_d);
-    put(lx, nxe, q_[2], nullptr, ws_[2], ws_[4], copy_d);
-    for (int q = 0; q < S_; ++q) put(lx, nxe, q_[3 + q], nullptr, ws_[8 + 3 * q], ws_[6 + 3 * q], copy_d);
+    put_d(q_[1], ws_[1], ws_[5]);
+    put_d(q_[2], ws_[2], ws_[4]);
+    for (int q = 0; q < S_; ++q) put_d(q_[3 + q], ws_[8 + 3 * q], ws_[6 + 3 * q]);
     put(ly, nye, ws_[0], ws_[5], ws_[0], ws_[5], curl_z);
     put(ly, nye, ws_[1], nullptr, ws_[1], nullptr, copy);
     put(ly, nye, ws_[2], nullptr, ws_[2], ws_[3], copy_d);
@@ -1637,7 +1653,6 @@ class Engine : public EngineBase {
       put(ly, nye, ws_[8 + 3 * q], nullptr, ws_[8 + 3 * q], ws_[7 + 3 * q], copy_d);
       put(ly, nye, ws_[6 + 3 * q], nullptr, ws_[6 + 3 * q], nullptr, copy);
     }
-    const int CC = pair_chunk(), CY = yc_ ? yc_ : CC;
     ColArgs ax;
     ax.estride = (long long)ny_ * kzs_;
     ax.ostride = kzs_;
@@ -1972,7 +1987,7 @@ class Engine : public EngineBase {
   double *dkx_ = nullptr, *dky_ = nullptr, *dkz_ = nullptr;
   T *tkx_ = nullptr, *tky_ = nullptr, *tkz_ = nullptr;
   double *d_part_ = nullptr, *d_spec_ = nullptr, *d_prof_ = nullptr, *d_cmax_ = nullptr, *d_fin_ = nullptr;
-  int* d_flag_ = nullptr;
+  int* flag_ = nullptr;  // a word of link_'s pinned memory
   void* scratch_ = nullptr;
   size_t scratch_n_ = 0;
   std::vector<void*> allocs_;

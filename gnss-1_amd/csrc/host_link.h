@@ -27,13 +27,15 @@ class HostLink {
   static constexpr size_t SLOT = 2u << 20;  // bytes of a slot: a large page, and 40 us of the bus
   static constexpr int SLOTS = 8;
 
-  // Pinned memory for transfers of up to `most` bytes at a time: as many slots as such a transfer fills.
+  // Pinned memory for transfers of up to `most` bytes at a time: as many slots as such a transfer fills, and
+  // one word beside them (flag()).
   void allocate(int dev, size_t most) {
     dev_ = dev;
     n_ = (int)std::min<size_t>(SLOTS, std::max<size_t>(1, (most + SLOT - 1) / SLOT));
     const size_t bytes = n_ == 1 ? std::max<size_t>(most, 1) : n_ * SLOT;
     slot_ = n_ == 1 ? bytes : SLOT;
-    if (hipHostMalloc(&base_, bytes, hipHostMallocDefault) != hipSuccess) {
+    flag_at_ = (bytes + 63) / 64 * 64;
+    if (hipHostMalloc(&base_, flag_at_ + 64, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       base_ = nullptr;
       throw Error(GNSS_ERR_ALLOC, "hipHostMalloc of " + std::to_string(bytes) + " bytes failed");
@@ -48,6 +50,7 @@ class HostLink {
     base_ = nullptr;
   }
   size_t slot_bytes() const { return slot_; }
+  int* flag() const { return reinterpret_cast<int*>((char*)base_ + flag_at_); }
 
   // fn(chunk, slot memory, the slot's event) for every chunk, on up to one thread per slot; the caller's
   // thread takes part.  An exception stops the chunks not yet begun and is thrown here.
@@ -79,7 +82,7 @@ class HostLink {
 
  private:
   int dev_ = 0, n_ = 0;
-  size_t slot_ = 0;
+  size_t slot_ = 0, flag_at_ = 0;
   void* base_ = nullptr;
   hipEvent_t ev_[SLOTS] = {};
 };

@@ -246,25 +246,9 @@ __global__ void k_ic_scatter(const IcEntry* __restrict__ e, int n, CPtrs<T> q) {
 
 // ---------------------------------------------------------------------------------------------
 // Statistics: deterministic FP64 reductions (fixed per-thread order + fixed tree), one block per
-// kx plane; the host sums the per-plane partials in plane order.
+// kx plane; the per-plane partials are summed in plane order.
 // ---------------------------------------------------------------------------------------------
 constexpr int STAT_THREADS = 256;
-
-// Fixed-order tree sum of NQ per-thread values over the block; every thread receives all NQ
-// totals in `out` (registers).  Reuses `sh`, so it starts with a barrier.
-template <int NQ>
-__device__ __forceinline__ void block_sum(const double (&acc)[NQ], double* sh, double (&out)[NQ]) {
-  const int tid = threadIdx.x;
-  __syncthreads();
-  for (int qq = 0; qq < NQ; ++qq) sh[qq * STAT_THREADS + tid] = acc[qq];
-  __syncthreads();
-  for (int s = STAT_THREADS / 2; s > 0; s >>= 1) {
-    if (tid < s)
-      for (int qq = 0; qq < NQ; ++qq) sh[qq * STAT_THREADS + tid] += sh[qq * STAT_THREADS + tid + s];
-    __syncthreads();
-  }
-  for (int qq = 0; qq < NQ; ++qq) out[qq] = sh[qq * STAT_THREADS];
-}
 
 constexpr int SPEC_NQ = 4 + 2 * 4;
 
@@ -585,15 +569,14 @@ k_plane_stats(Geom g, RPtrs<T> ph, int S, double idx_, double idy_, double idz_,
   }
 }
 
-// Any non-finite value in the kz = 0 column of a field (cheap NaN/Inf watchdog after a step).
+// Any non-finite value in the kz = 0 column of field blockIdx.y (cheap NaN/Inf watchdog after a step); the flag
+// is in pinned host memory, which the host has cleared.
 template <typename T>
-__global__ void k_finite(Geom g, CPtrs<T> q, int F, int* __restrict__ flag) {
+__global__ void k_finite(Geom g, CPtrs<T> q, int* __restrict__ flag) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (long long)g.nx * g.ny) return;
-  for (int f = 0; f < F; ++f) {
-    const cx<T> v = q.p[f][i * g.kzs];
-    if (!isfinite((double)v.x) || !isfinite((double)v.y)) flag[0] = 1;
-  }
+  const cx<T> v = q.p[blockIdx.y][i * g.kzs];
+  if (!isfinite((double)v.x) || !isfinite((double)v.y)) flag[0] = 1;
 }
 
 
@@ -1158,25 +1141,25 @@ static __global__ void __launch_bounds__(256) k_copy16(const v4f* __restrict__ i
 // Diagnostics
 // ---------------------------------------------------------------------------------------------
 
-// omega^ = i k x u^ over the whole spectral array (calcOmega*Kernel_mgpu, solver.cu:68-114);
-// the kz padding is written as zero.
+// omega^ = i k x u^ (calcOmega*Kernel_mgpu, solver.cu:68-114) over a box of modes: the whole array, whose
+// kz padding is written as zero, or the kept box of a dealiased state.
 template <typename T>
-__global__ void k_vorticity(Geom g, CPtrs<T> q, CPtrs<T> w, const T* __restrict__ kxv,
+__global__ void k_vorticity(Geom g, Box b, CPtrs<T> q, CPtrs<T> w, const T* __restrict__ kxv,
                             const T* __restrict__ kyv, const T* __restrict__ kzv, long long n) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int iz = (int)(i % g.kzs);
-  const long long r = i / g.kzs;
-  const int iy = (int)(r % g.ny), ix = (int)(r / g.ny);
+  int ix, iy, iz;
+  box_index(g, b, i, ix, iy, iz);
+  const long long o = ((long long)ix * g.ny + iy) * g.kzs + iz;
   if (iz >= g.nzh) {
-    for (int c = 0; c < 3; ++c) w.p[c][i] = mk<T>(0, 0);
+    for (int c = 0; c < 3; ++c) w.p[c][o] = mk<T>(0, 0);
     return;
   }
   const T kx = kxv[ix], ky = kyv[iy], kz = kzv[iz];
-  const cx<T> u = q.p[0][i], v = q.p[1][i], ww = q.p[2][i];
-  w.p[0][i] = csub(ik(ky, ww), ik(kz, v));
-  w.p[1][i] = csub(ik(kz, u), ik(kx, ww));
-  w.p[2][i] = csub(ik(kx, v), ik(ky, u));
+  const cx<T> u = q.p[0][o], v = q.p[1][o], ww = q.p[2][o];
+  w.p[0][o] = csub(ik(ky, ww), ik(kz, v));
+  w.p[1][o] = csub(ik(kz, u), ik(kx, ww));
+  w.p[2][o] = csub(ik(kx, v), ik(ky, u));
 }
 
 // |(a, b, c)| in place over a (VectorMagnitude_kernel, statistics.cu:2005-2018).
@@ -1210,33 +1193,53 @@ __global__ void k_plane(const T* __restrict__ a, double* __restrict__ out, int n
 
 // Iso-surface area by the indicator gradient (surfaceArea_kernel_mgpu, statistics.cu:1310-1460):
 // per grid point -(grad F . grad chi) / |grad F| with chi = (F <= iso), central differences on the
-// periodic grid; one block per x plane, fixed per-thread order and tree -> part[x] (FP64).
+// periodic grid; AREA_SPLIT blocks per x plane, each with every AREA_SPLIT-th group of rows, fixed per-thread
+// order and tree -> part[x AREA_SPLIT + block] (FP64).  A thread takes 16 bytes of z; away from the surface
+// the indicator has no gradient and nothing but the comparisons is computed.  Bound by reading F.
+constexpr int AREA_SPLIT = 4;
+constexpr int AREA_THREADS = 512;
 template <typename T>
-__global__ void __launch_bounds__(STAT_THREADS)
+__global__ void __launch_bounds__(AREA_THREADS)
 k_surface_area(Geom g, const T* __restrict__ F, double iso, double dx, double dy, double dz,
                double* __restrict__ part) {
-  __shared__ double sh[STAT_THREADS];
+  constexpr int V = 16 / (int)sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(V)));
+  __shared__ double sh[AREA_THREADS / 64];
   const int x = blockIdx.x;
   const int xm = x == 0 ? g.nx - 1 : x - 1, xp = x == g.nx - 1 ? 0 : x + 1;
-  const long long plane = (long long)g.ny * g.nz;
-  double acc[1] = {0.0};
-  for (long long i = threadIdx.x; i < plane; i += STAT_THREADS) {
-    const int y = (int)(i / g.nz), z = (int)(i % g.nz);
+  const int nv = g.nz / V, n = g.ny * nv;
+  const vec* __restrict__ Fv = reinterpret_cast<const vec*>(F);
+  double acc = 0.0;
+  for (int i = blockIdx.y * AREA_THREADS + threadIdx.x; i < n; i += AREA_SPLIT * AREA_THREADS) {
+    const int y = i / nv, zv = i - y * nv;
     const int ym = y == 0 ? g.ny - 1 : y - 1, yp = y == g.ny - 1 ? 0 : y + 1;
-    const int zm = z == 0 ? g.nz - 1 : z - 1, zp = z == g.nz - 1 ? 0 : z + 1;
-    auto at = [&](int a, int b, int c) { return (double)F[((long long)a * g.ny + b) * g.nz + c]; };
-    const double fxm = at(xm, y, z), fxp = at(xp, y, z), fym = at(x, ym, z), fyp = at(x, yp, z);
-    const double fzm = at(x, y, zm), fzp = at(x, y, zp);
-    const double gx = (fxp - fxm) / (2.0 * dx), gy = (fyp - fym) / (2.0 * dy), gz = (fzp - fzm) / (2.0 * dz);
-    const double cxv = ((double)(fxp <= iso) - (double)(fxm <= iso)) / (2.0 * dx);
-    const double cyv = ((double)(fyp <= iso) - (double)(fym <= iso)) / (2.0 * dy);
-    const double czv = ((double)(fzp <= iso) - (double)(fzm <= iso)) / (2.0 * dz);
-    if ((gx == 0 && gy == 0 && gz == 0) || (cxv == 0 && cyv == 0 && czv == 0)) continue;
-    acc[0] += -(gx * cxv + gy * cyv + gz * czv) / sqrt(gx * gx + gy * gy + gz * gz);
+    auto at = [&](int a, int b) { return ((long long)a * g.ny + b) * nv + zv; };
+    const vec c = Fv[at(x, y)], vxm = Fv[at(xm, y)], vxp = Fv[at(xp, y)], vym = Fv[at(x, ym)], vyp = Fv[at(x, yp)];
+    const long long row = ((long long)x * g.ny + y) * g.nz;
+    const T before = F[row + (zv == 0 ? g.nz - 1 : zv * V - 1)], after = F[row + (zv == nv - 1 ? 0 : zv * V + V)];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const double fxm = vxm[j], fxp = vxp[j], fym = vym[j], fyp = vyp[j];
+      const double fzm = j == 0 ? (double)before : (double)c[j > 0 ? j - 1 : 0];
+      const double fzp = j == V - 1 ? (double)after : (double)c[j < V - 1 ? j + 1 : 0];
+      const int ix = (int)(fxp <= iso) - (int)(fxm <= iso), iy = (int)(fyp <= iso) - (int)(fym <= iso);
+      const int iz = (int)(fzp <= iso) - (int)(fzm <= iso);
+      if (ix == 0 && iy == 0 && iz == 0) continue;
+      const double gx = (fxp - fxm) / (2.0 * dx), gy = (fyp - fym) / (2.0 * dy), gz = (fzp - fzm) / (2.0 * dz);
+      if (gx == 0 && gy == 0 && gz == 0) continue;
+      const double cxv = (double)ix / (2.0 * dx), cyv = (double)iy / (2.0 * dy), czv = (double)iz / (2.0 * dz);
+      acc += -(gx * cxv + gy * cyv + gz * czv) / sqrt(gx * gx + gy * gy + gz * gz);
+    }
   }
-  double tot[1];
-  block_sum<1>(acc, sh, tot);
-  if (threadIdx.x == 0) part[x] = tot[0];
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) acc += __shfl_down(acc, d);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < AREA_THREADS / 64; ++w) t += sh[w];
+    part[x * AREA_SPLIT + blockIdx.y] = t;
+  }
 }
 
 }  // namespace gnss
