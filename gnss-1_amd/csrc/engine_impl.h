@@ -432,14 +432,7 @@ class Engine : public EngineBase {
   void get_field(int f, int space, double* host) override {
     check_field(f);
     if (space == GNSS_PHYSICAL) {
-      const long long per = (long long)(link_.slot_bytes() / sizeof(T)) / 4 * 4;
-      link_.each((int)cdiv(nph_, per), [&](int c, void* mem, hipEvent_t ev) {
-        const long long i0 = c * per, n = std::min(per, nph_ - i0);
-        hipLaunchKernelGGL(k_real_copy<T>, dim3(link_grid(n / 4)), dim3(256), 0, s_, phys_[f] + i0, (T*)mem, n / 4);
-        launch_done("k_real_copy", ev);
-        GNSS_HIP(hipEventSynchronize(ev));
-        widen((const T*)mem, host + i0, (size_t)n);
-      });
+      reals_to_host(phys_[f], nph_, (long long)(link_.slot_bytes() / sizeof(T)) / 4 * 4, host);
       return;
     }
     if (space != GNSS_SPECTRAL) throw Error(GNSS_ERR_ARG, "bad space");
@@ -641,13 +634,62 @@ class Engine : public EngineBase {
     const int n[3] = {nx_, ny_, nz_};
     if (axis < 0 || axis > 2 || index < 0 || index >= n[axis])
       throw Error(GNSS_ERR_ARG, "plane " + std::to_string(index) + " of axis " + std::to_string(axis) + " out of range");
-    const T* a = diag_field(field);
+    need_k();
     const long long np = axis == 2 ? (long long)nx_ * ny_ : (axis == 1 ? (long long)nx_ * nz_ : (long long)ny_ * nz_);
-    double* d = reinterpret_cast<double*>(ws_[2]);  // np doubles <= one complex work buffer
-    hipLaunchKernelGGL(k_plane<T>, dim3((unsigned)cdiv(np, 256)), dim3(256), 0, s_, a, d, nx_, ny_, nz_, axis, index);
-    GNSS_HIP(hipGetLastError());
-    GNSS_HIP(hipMemcpyAsync(host, d, sizeof(double) * np, hipMemcpyDeviceToHost, s_));
-    sync();
+    const long long per = (long long)(link_.slot_bytes() / sizeof(T)) / 4 * 4;
+    if (field == GNSS_FIELD_VORTICITY) {
+      const T* a = diag_field(field);
+      T* d = reinterpret_cast<T*>(ws_[2]);  // np values <= one complex work buffer
+      hipLaunchKernelGGL(k_plane<T>, dim3((unsigned)cdiv(np, 256)), dim3(256), 0, s_, a, d, nx_, ny_, nz_, axis, index);
+      check_launch("k_plane");
+      reals_to_host(d, np, per, host);
+      return;
+    }
+    if (field < 0 || field >= F_) throw Error(GNSS_ERR_ARG, "field " + std::to_string(field) + " out of range");
+    // summed over the axis first, then only the plane is transformed (512^3 FP32, z = const: 0.10 ms on the
+    // device where the inverse transform of the whole field took 0.45)
+    const C* q = q_[field];
+    C* h = ws_[0];
+    const T scale = (T)(1.0 / ((double)nx_ * ny_ * nz_));
+    const int nkz = clean_ ? std::min(g_.keep_z + 1, nzh_) : nzh_;
+    constexpr int CC = PLANE_COLS;
+    if (axis == 2) {
+      hipLaunchKernelGGL(k_sum_z<T>, dim3((unsigned)cdiv((long long)nx_ * ny_, 256 / PLANE_COLS)), dim3(256), 0, s_, g_,
+                         q, h, tw_.at(nz_), index, clean_ ? 1 : 0, nkz);
+      check_launch("k_sum_z");
+      plane_pass(h, nx_, (long long)ny_ * PLANE_COLS, PLANE_COLS, ny_, 1, CC);
+      plane_pass(h, ny_, PLANE_COLS, (long long)ny_ * PLANE_COLS, nx_, 1, CC);
+      link_.each((int)cdiv(np, per), [&](int c, void* mem, hipEvent_t ev) {
+        const long long i0 = c * per, n = std::min(per, np - i0);
+        hipLaunchKernelGGL(k_plane_out<T>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s_, h, (T*)mem, i0, n, scale);
+        launch_done("k_plane_out", ev);
+        GNSS_HIP(hipEventSynchronize(ev));
+        widen((const T*)mem, host + i0, (size_t)n);
+      });
+      return;
+    }
+    const int na = axis == 1 ? nx_ : ny_;
+    const unsigned grid = (unsigned)cdiv((long long)na * kzs_, 256);
+    if (axis == 1)
+      hipLaunchKernelGGL((k_sum_xy<T, 1>), dim3(grid), dim3(256), 0, s_, g_, q, h, tw_.at(ny_), index,
+                         clean_ ? g_.keep_y : -1, nkz);
+    else
+      hipLaunchKernelGGL((k_sum_xy<T, 0>), dim3(grid), dim3(256), 0, s_, g_, q, h, tw_.at(nx_), index,
+                         clean_ ? g_.keep_x : -1, nkz);
+    check_launch("k_sum_xy");
+    plane_pass(h, na, kzs_, 0, 1, kzs_ / CC, CC);
+    T* d = reinterpret_cast<T*>(ws_[1]);
+    z_c2r(&h, &d, 1, nzh_, scale, na);
+    reals_to_host(d, np, per, host);
+  }
+  void reals_to_host(const T* d, long long np, long long per, double* host) {
+    link_.each((int)cdiv(np, per), [&](int c, void* mem, hipEvent_t ev) {
+      const long long i0 = c * per, n = std::min(per, np - i0);
+      hipLaunchKernelGGL(k_real_copy<T>, dim3(link_grid(n / 4)), dim3(256), 0, s_, d + i0, (T*)mem, n / 4);
+      launch_done("k_real_copy", ev);
+      GNSS_HIP(hipEventSynchronize(ev));
+      widen((const T*)mem, host + i0, (size_t)n);
+    });
   }
 
   double surface_area(int field, double iso) override {
@@ -1372,6 +1414,25 @@ class Engine : public EngineBase {
     }
   }
 
+  // An inverse pass of length L along `estride` over whole columns of one array (planes), CC columns a tile.
+  void plane_pass(C* data, int L, long long estride, long long ostride, int nouter, int nchunks, int CC) {
+    const int TPC = L / elems_per_thread(L);
+    ColArgs a;
+    a.estride = estride;
+    a.ostride = ostride;
+    a.nouter = nouter;
+    a.outer_keep = -1;
+    a.outer_n = nouter;
+    a.nchunks = nchunks;
+    a.in_keep = a.out_keep = -1;
+    int G = std::max(1, 256 / (CC * TPC));
+    while (G > 1 && (long long)G * L * CC * (long long)sizeof(C) > LDS_MAX) --G;
+    a.G = G;
+    FieldList<T> fl{};
+    fl.in[0] = fl.p[0] = data;
+    timed("fft_plane", 2.0 * nouter * nchunks * CC * L * sizeof(C), [&] { col_dispatch_l<+1>(L, fl, 1, a, CC, G, 1); });
+  }
+
   template <int NZ>
   void zr2c_launch(const T* in, C* out, int out_lim) {
     constexpr int M = NZ / 2;
@@ -1391,12 +1452,11 @@ class Engine : public EngineBase {
                        tw_.at(M), tw_.at(NZ), rows, kzs_, out_lim, G);
   }
   template <int NZ>
-  void zc2r_launch(const ZList<T>& zl, int nf, int in_lim, T scale) {
+  void zc2r_launch(const ZList<T>& zl, int nf, int in_lim, T scale, long long rows) {
     constexpr int M = NZ / 2;
     constexpr int TPC = M / Plan<M>::E;
     int G = std::max(1, 256 / TPC);
     while (G > 1 && (long long)G * zrow_stride(M) * (long long)sizeof(C) > LDS_MAX) --G;
-    const long long rows = (long long)nx_ * ny_;
     const size_t lds = (size_t)G * zrow_stride(M) * sizeof(C);
     if (zp_) {
       const long long groups = cdiv(rows, G);
@@ -1439,14 +1499,15 @@ class Engine : public EngineBase {
     timed("fft_z_r2c", bytes, [&] { GNSS_Z_SWITCH(zr2c_launch, in, out, out_lim); });
   }
   void z_c2r(const C* in, T* out, int in_lim, T scale) { z_c2r(&in, &out, 1, in_lim, scale); }
-  void z_c2r(const C* const* in, T* const* out, int nf, int in_lim, T scale) {
+  void z_c2r(const C* const* in, T* const* out, int nf, int in_lim, T scale, long long rows = 0) {
+    if (rows == 0) rows = (long long)nx_ * ny_;
     ZList<T> zl{};
     for (int f = 0; f < nf; ++f) {
       zl.in[f] = in[f];
       zl.out[f] = out[f];
     }
-    const double bytes = (double)nf * nx_ * ny_ * ((double)nz_ * sizeof(T) + (double)std::min(in_lim, nzh_) * sizeof(C));
-    timed("fft_z_c2r", bytes, [&] { GNSS_Z_SWITCH(zc2r_launch, zl, nf, in_lim, scale); });
+    const double bytes = (double)nf * rows * ((double)nz_ * sizeof(T) + (double)std::min(in_lim, nzh_) * sizeof(C));
+    timed("fft_z_c2r", bytes, [&] { GNSS_Z_SWITCH(zc2r_launch, zl, nf, in_lim, scale, rows); });
   }
 
   // Forward 3D R2C: in (physical) -> out (spectral).  prune: only the kept box is produced.

@@ -1171,10 +1171,10 @@ __global__ void k_magnitude(T* __restrict__ a, const T* __restrict__ b, const T*
   a[i] = sqrt(x * x + y * y + z * z);
 }
 
-// One physical plane [x][y][z] -> FP64: axis 2 (z = index) -> [x][y], axis 1 -> [x][z],
+// One physical plane of [x][y][z]: axis 2 (z = index) -> [x][y], axis 1 -> [x][z],
 // axis 0 -> [y][z] (writexyfields / writexzfields / writeyzfields, iofuncs.cu:187-260).
 template <typename T>
-__global__ void k_plane(const T* __restrict__ a, double* __restrict__ out, int nx, int ny, int nz, int axis,
+__global__ void k_plane(const T* __restrict__ a, T* __restrict__ out, int nx, int ny, int nz, int axis,
                         int index) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   long long src;
@@ -1188,7 +1188,83 @@ __global__ void k_plane(const T* __restrict__ a, double* __restrict__ out, int n
     if (i >= (long long)ny * nz) return;
     src = (long long)index * ny * nz + i;
   }
-  out[i] = (double)a[src];
+  out[i] = a[src];
+}
+
+// A plane of a field at one index of an axis is linear in the spectrum: summed over that axis' modes
+// first, what is left to transform is a plane.  The sums are taken in FP64 (twiddles from the passes' tables)
+// and read the state once, or its kept modes only (kept != 0: a dealiased state).
+
+// z = index: h[kx][ky][0] = sum over kz, weighted so that the real part of the plane's transform is the field
+// (2 for the modes whose conjugates the half spectrum leaves out); columns 1 to 7 are zeros (a column tile).  A
+// row is summed by the 8 lanes that write its columns: 64 bytes a load in FP32, and the table index goes round by
+// addition (a wave per row and a remainder per mode: 25 us at 256x384x192 FP32, now 12).
+constexpr int PLANE_COLS = 8;
+template <typename T>
+__global__ void __launch_bounds__(256) k_sum_z(Geom g, const cx<T>* __restrict__ q, cx<T>* __restrict__ h,
+                                               const cx<T>* __restrict__ tw, int index, int kept_only, int nkz) {
+  const int lane = threadIdx.x % PLANE_COLS;
+  const long long r = (long long)blockIdx.x * (256 / PLANE_COLS) + threadIdx.x / PLANE_COLS;
+  if (r >= (long long)g.nx * g.ny) return;
+  const int ix = (int)(r / g.ny), iy = (int)(r % g.ny);
+  double re = 0.0, im = 0.0;
+  if (!kept_only || kept(g, mode_of(ix, g.nx), mode_of(iy, g.ny), 0)) {
+    const cx<T>* row = q + r * g.kzs;
+    int at = (int)((unsigned)(lane * index) % (unsigned)g.nz);
+    const int by = (int)((unsigned)(PLANE_COLS * index) % (unsigned)g.nz);
+#pragma unroll 4
+    for (int k = lane; k < nkz; k += PLANE_COLS) {
+      const cx<T> f = row[k], w = tw[at];
+      const double s = (k == 0 || 2 * k == g.nz) ? 1.0 : 2.0;
+      re += s * ((double)f.x * w.x + (double)f.y * w.y);
+      im += s * ((double)f.y * w.x - (double)f.x * w.y);
+      at += by;
+      at -= at >= g.nz ? g.nz : 0;
+    }
+#pragma unroll
+    for (int d = PLANE_COLS / 2; d > 0; d >>= 1) {
+      re += __shfl_xor(re, d, PLANE_COLS);
+      im += __shfl_xor(im, d, PLANE_COLS);
+    }
+  }
+  h[r * PLANE_COLS + lane] = lane == 0 ? mk<T>((T)re, (T)im) : mk<T>(0, 0);
+}
+
+// y = index (AXIS 1: a runs over kx, the sum over ky) or x = index (AXIS 0: a over ky, the sum over kx):
+// h[a][kz], zeros from kz = nkz on.  A thread per (a, kz), keep: the sum's largest kept |mode|, or -1.
+template <typename T, int AXIS>
+__global__ void __launch_bounds__(256) k_sum_xy(Geom g, const cx<T>* __restrict__ q, cx<T>* __restrict__ h,
+                                                const cx<T>* __restrict__ tw, int index, int keep, int nkz) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int na = AXIS ? g.nx : g.ny, n = AXIS ? g.ny : g.nx;
+  if (i >= (long long)na * g.kzs) return;
+  const int a = (int)(i / g.kzs), k = (int)(i % g.kzs);
+  double re = 0.0, im = 0.0;
+  if (k < nkz) {
+    const int nm = keep < 0 ? n : 2 * keep + 1;
+    // the modes in order from 0, or from -keep: the table index goes round by addition
+    int m = keep < 0 ? 0 : n - keep, at = (int)((unsigned)(m * index) % (unsigned)n);
+    if (keep == 0) m = 0;
+#pragma unroll 4
+    for (int o = 0; o < nm; ++o) {
+      const long long row = AXIS ? (long long)a * g.ny + m : (long long)m * g.ny + a;
+      const cx<T> f = q[row * g.kzs + k], w = tw[at];
+      m = m + 1 == n ? 0 : m + 1;
+      at += index;
+      at -= at >= n ? n : 0;
+      re += (double)f.x * w.x + (double)f.y * w.y;
+      im += (double)f.y * w.x - (double)f.x * w.y;
+    }
+  }
+  h[i] = mk<T>((T)re, (T)im);
+}
+
+// The real parts of column 0 of a z plane, from point i0 on, times `scale`, to (pinned host) memory.
+template <typename T>
+__global__ void __launch_bounds__(256) k_plane_out(const cx<T>* __restrict__ h, T* __restrict__ out, long long i0,
+                                                   long long n, T scale) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = h[(i0 + i) * PLANE_COLS].x * scale;
 }
 
 // Iso-surface area by the indicator gradient (surfaceArea_kernel_mgpu, statistics.cu:1310-1460):
