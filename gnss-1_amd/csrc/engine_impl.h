@@ -69,6 +69,7 @@ class Engine : public EngineBase {
     mask_factors(nx_, ny_, nz_, ax, ay, az, g2);
     g_.ax = ax; g_.ay = ay; g_.az = az; g_.g2 = g2;
     kz_lim_ = std::min(round_up(g_.keep_z + 1, cmax), kzs_);
+    kz_cols_ = zfused_lim<T>(nz_);
     sph_.shift = sizeof(T) == 8 ? 3 : 4;  // cmax
     sph_.r2 = (float)((double)g_.g2 / 9.0);
     sph_.ay = (float)g_.ay;
@@ -1253,6 +1254,7 @@ class Engine : public EngineBase {
     int nchunks;     // column chunks processed
     int outer_keep;  // kept-mode outer map (x pass: over ky), -1 = all
     int in_keep, out_keep;
+    int cols = 0;    // columns in use (0: whole tiles)
     bool pruned() const { return in_keep >= 0 || out_keep >= 0; }
   };
 
@@ -1380,6 +1382,7 @@ class Engine : public EngineBase {
     a.nchunks = sp.nchunks;
     a.in_keep = sp.in_keep;
     a.out_keep = sp.out_keep;
+    a.cols = sp.cols ? sp.cols : sp.nchunks * CC;
     if (sp.pruned()) a.sph = sphere(sp.axis);
     batch_outer(a);
     int G = std::max(1, 256 / (CC * TPC));
@@ -1424,6 +1427,7 @@ class Engine : public EngineBase {
     a.outer_keep = -1;
     a.outer_n = nouter;
     a.nchunks = nchunks;
+    a.cols = nchunks * CC;
     a.in_keep = a.out_keep = -1;
     int G = std::max(1, 256 / (CC * TPC));
     while (G > 1 && (long long)G * L * CC * (long long)sizeof(C) > LDS_MAX) --G;
@@ -1691,7 +1695,7 @@ class Engine : public EngineBase {
     // Small grids take a field and its x derivative in blocks of their own (the passes' outputs are not their
     // inputs): the launch then lasts one transform instead of two.
     const int CC = pair_chunk(), CY = yc_ ? yc_ : CC;
-    const long long xtiles = (long long)(kz_lim_ / CC) * (2 * g_.keep_y + 1) * bm_ * (3 + S_);
+    const long long xtiles = (long long)kz_tiles(CC) * (2 * g_.keep_y + 1) * bm_ * (3 + S_);
     const bool apart = xtiles * (CC * nx_ / elems_per_thread(nx_)) <= (long long)n_cu_ * 1024;
     const PairOp deriv{1, 1, {0, 0}, {1, 0}, {0, 0}, {0, 0}};       // out0 = i k A
     auto put_d = [&](const C* A, C* o0, C* o1) {
@@ -1720,7 +1724,8 @@ class Engine : public EngineBase {
     ax.outer_keep = g_.keep_y;
     ax.outer_n = ny_;
     ax.nouter = 2 * g_.keep_y + 1;
-    ax.nchunks = kz_lim_ / CC;
+    ax.nchunks = kz_tiles(CC);
+    ax.cols = kz_cols_;
     ax.in_keep = g_.keep_x;
     ax.out_keep = -1;
     ax.G = 1;
@@ -1731,7 +1736,8 @@ class Engine : public EngineBase {
     ay.outer_keep = -1;
     ay.outer_n = nx_;
     ay.nouter = nx_;
-    ay.nchunks = kz_lim_ / CY;
+    ay.nchunks = kz_tiles(CY);
+    ay.cols = kz_cols_;
     ay.in_keep = g_.keep_y;
     ay.out_keep = -1;
     ay.G = 1;
@@ -1742,6 +1748,7 @@ class Engine : public EngineBase {
     pair_pass(ly, nye, ay, ny_, tky_, "fft_y_inv_late", CY);
   }
   int pair_chunk() const { return xc_; }
+  int kz_tiles(int cc) const { return (kz_cols_ + cc - 1) / cc; }  // column tiles of a substage's passes
   // The 2/3 rule's ellipsoid for a pruned pass over kx (axis 0) or ky (1) rows.  Off for the MFMA
   // passes, which read and write whole boxes.
   Sphere sphere(int axis) const {
@@ -1834,7 +1841,8 @@ class Engine : public EngineBase {
     a.outer_keep = g_.keep_y;
     a.outer_n = ny_;
     a.nouter = 2 * g_.keep_y + 1;
-    a.nchunks = kz_lim_ / xc_;
+    a.nchunks = kz_tiles(xc_);
+    a.cols = kz_cols_;
     a.in_keep = g_.keep_x;
     a.out_keep = -1;
     a.sph = sphere(0);
@@ -1903,7 +1911,7 @@ class Engine : public EngineBase {
     int G = std::max(1, 256 / (CC * TPC));
     const long long twb = pro ? 0 : (long long)L * (long long)(sizeof(C) + sizeof(T));
     while (G > 1 && (long long)G * L * CC * (long long)sizeof(C) + twb > LDS_MAX) --G;
-    const int nchunks = kz_lim_ / CC;
+    const int nchunks = kz_tiles(CC);
     const int nouter = 2 * g_.keep_y + 1;
     const double kept_rows = 2 * g_.keep_x + 1;
     const bool cgrp = pro && colloid_ && grp == S_ - 1;
@@ -1943,11 +1951,8 @@ class Engine : public EngineBase {
     a.alpha = (T)p_.alpha;
     a.late = ((p_.flags & GNSS_FLAG_UNFUSED) == 0 && x_mode() >= 4) ? 1 : 0;
     a.kz = tkz_;
-    if (kz_lim_ != zfused_lim<T>(nz_))
-      throw Error(GNSS_ERR_UNSUPPORTED, "fused z pass: pruned kz limit " + std::to_string(kz_lim_) + " differs from " +
-                                            std::to_string(zfused_lim<T>(nz_)));
     const T scale = (T)(1.0 / ((double)nx_ * ny_ * nz_));
-    const double bytes = (double)bm_ * nx_ * ny_ * (double)kz_lim_ * sizeof(C) * (W_ + F_);
+    const double bytes = (double)bm_ * nx_ * ny_ * (double)kz_cols_ * sizeof(C) * (W_ + F_);
     timed("fft_z_fused", bytes, [&] { GNSS_Z_SWITCH(zfused_launch, a, scale); });
   }
 
@@ -2000,12 +2005,12 @@ class Engine : public EngineBase {
         late_inverse();
       } else {
         if (xm >= 2) x_inv_ops();
-        else if (xm == 0) col_passes(ws_.data(), W_, ColSpec{0, +1, kz_lim_ / cx_, g_.keep_y, g_.keep_x, -1});
-        col_passes(ws_.data(), W_, ColSpec{1, +1, kz_lim_ / cy_, -1, g_.keep_y, -1});
+        else if (xm == 0) col_passes(ws_.data(), W_, ColSpec{0, +1, kz_tiles(cx_), g_.keep_y, g_.keep_x, -1, kz_cols_});
+        col_passes(ws_.data(), W_, ColSpec{1, +1, kz_tiles(cy_), -1, g_.keep_y, -1, kz_cols_});
       }
       z_fused();
-      col_passes(nl_.data(), F_, ColSpec{1, -1, kz_lim_ / cy_, -1, -1, g_.keep_y});
-      if (!xfwd) col_passes(nl_.data(), F_, ColSpec{0, -1, kz_lim_ / cx_, g_.keep_y, -1, g_.keep_x});
+      col_passes(nl_.data(), F_, ColSpec{1, -1, kz_tiles(cy_), -1, -1, g_.keep_y, kz_cols_});
+      if (!xfwd) col_passes(nl_.data(), F_, ColSpec{0, -1, kz_tiles(cx_), g_.keep_y, -1, g_.keep_x, kz_cols_});
     }
     if (xfwd) {
       x_fused(false, -1, c);
@@ -2013,15 +2018,18 @@ class Engine : public EngineBase {
       return;
     }
     RkCoef cm = c;
+    Box br = b;
+    br.bz = kz_cols_;
+    const long long nr = (long long)br.bx * br.by * br.bz;
     if (bm_ > 1) {
-      cm.nbox = nb;
+      cm.nbox = nr;
       cm.mstride = nsp_;
       cm.nu_m = d_num_;
     }
-    const long long n = nb * bm_;
+    const long long n = nr * bm_;
     const double rk_bytes = (double)n * F_ * sizeof(C) * (c.first ? 3 : (c.last ? 4 : 5));
     timed("k_rk", rk_bytes, [&] {
-      hipLaunchKernelGGL(k_rk<T>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s_, g_, b, ptrs(q_), ptrs(dq_),
+      hipLaunchKernelGGL(k_rk<T>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s_, g_, br, ptrs(q_), ptrs(dq_),
                          ptrs(nl_), tkx_, tky_, tkz_, cm, F_, n);
     });
   }
@@ -2037,7 +2045,8 @@ class Engine : public EngineBase {
   std::vector<gnss_params> mp_;
   std::vector<C*> qb_, dqb_;
   double* d_num_ = nullptr;
-  int kz_lim_ = 0;
+  int kz_lim_ = 0;   // kz entries the strided passes' tiles cover: the kept modes and up to a tile more
+  int kz_cols_ = 0;  // of those, what a substage's passes move (zfused_lim)
   long long nsp_ = 0, nph_ = 0;
   Geom g_{};
   Sphere sph_{};

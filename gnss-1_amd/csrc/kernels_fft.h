@@ -73,6 +73,7 @@ struct ColArgs {
   int nouter_m = 0;    // batched contexts: outer indices per member (0: one member)
   long long mstride = 0;  // batched contexts: elements between members
   Sphere sph{};        // bounds of the 2/3 rule's ellipsoid, for pruned passes (axis < 0: none)
+  int cols = 0;        // columns in use: those of the last tile from here on are neither read nor written
 };
 
 // What one tile of a strided pass has to do under the ellipsoid: nothing (dead: an x pass's column of
@@ -134,6 +135,7 @@ k_col(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a) {
   const TileRows in = tile_rows(a.sph, io, a.outer_n, chunk * C, a.in_keep);
   active = active && in.live;
   if (a.G == 1 && !active) return;
+  active = active && chunk * C + c < a.cols;
   cx<T>* twl = lds + (long long)a.G * L * C;
   for (int i = tid; i < L; i += blockDim.x) twl[i] = tw[i];
   const long long off = mo + (long long)io * a.ostride + (long long)chunk * C + c;
@@ -184,6 +186,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
     r.live = r.live && active;
     return mo + (long long)io * a.ostride + (long long)chunk * C + c;
   };
+  auto in_use = [&](int tile) { return tile % tpf % a.nchunks * C + c < a.cols; };
   // with one group per block the removed columns are passed over
   auto live_from = [&](int tile) {
     if (a.G == 1 && a.sph.axis == 0) {
@@ -198,6 +201,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
   auto load = [&](int tile, cx<T>* v) {
     TileRows r;
     const cx<T>* base = fl.in[tile / tpf] + off_of(tile, r, a.in_keep);
+    r.live = r.live && in_use(tile);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = t + e * TPC;
@@ -230,7 +234,7 @@ k_col_multi(FieldList<T> fl, const cx<T>* __restrict__ tw, ColArgs a, int tpf, i
     wait_vmem();
     TileRows r;
     cx<T>* base = fl.p[tile / tpf] + off_of(tile, r, a.out_keep);
-    if (r.live) {
+    if (r.live && in_use(tile)) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int p = t + e * TPC;
@@ -685,10 +689,13 @@ template <typename T, int M> struct FusedPlan<T, M, 9> {
 // V = 10: variant 9 with a colloid.
 template <typename T, int M> struct FusedPlan<T, M, 10> : FusedPlan<T, M, 9> {};
 
-// kz entries a substage's rows hold: kz <= nz/3 (the 2/3 rule), rounded up to the widest column tile
-// of the strided passes (16 complex in FP32, 8 in FP64); the engine's pruned kz limit.
+// kz entries a substage's rows hold: kz <= nz/3 (the 2/3 rule), rounded up to 64 bytes.  Rounded up to the strided
+// passes' widest tiles (128 bytes), FP32 rows of 96 held 48 entries for 33 modes, now 40: 1024 x 128 x 96, the
+// fused z pass 165 -> 153 us, the update 54 -> 44, a substage 448 -> 430.  The strided passes of 16-column
+// tiles, which leave half of the last one alone, gain nothing from it (192^3 y inverse 66.0 -> 65.6 us).
 template <typename T> __host__ __device__ constexpr int zfused_lim(int nz) {
-  return (nz / 3 + 1 + (sizeof(T) == 8 ? 7 : 15)) / (sizeof(T) == 8 ? 8 : 16) * (sizeof(T) == 8 ? 8 : 16);
+  constexpr int S = 64 / (int)sizeof(cx<T>);
+  return (nz / 3 + 1 + S - 1) / S * S;
 }
 
 template <typename T> struct ZFusedArgs {

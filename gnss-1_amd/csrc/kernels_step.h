@@ -722,7 +722,7 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int p = t + e * TPC;
-      const bool ld = r.live && row_kept(p, L, r.keep);
+      const bool ld = r.live && iz < a.cols && row_kept(p, L, r.keep);
       va[e] = ld ? ld_s(&src[off + (long long)p * a.estride]) : mk<T>(0, 0);
     }
   };
@@ -762,7 +762,7 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
     TileRows r;
     int iy, iz;
     const long long off = offset_of(tile, r, iy, iz);
-    if (r.live) {
+    if (r.live && iz < a.cols) {
       cx<T>* __restrict__ out = li.out[tile / tpf];
 #pragma unroll
       for (int e = 0; e < E; ++e) st_s(&out[off + (long long)(t + e * TPC) * a.estride], v[e]);
@@ -850,6 +850,7 @@ k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ t
   TileRows r;
   const long long off = tile_off(blockIdx.x, r);
   if (a.G == 1 && !r.live) return;
+  r.live = r.live && (int)(blockIdx.x % tpf % a.nchunks) * C + c < a.cols;
   for (int i = tid; i < L; i += blockDim.x) {
     twl[i] = tw[i];
     kl[i] = kv[i];
@@ -947,7 +948,8 @@ k_xfwd_rk(Geom g, CPtrs<T> q, CPtrs<T> dq, CPtrs<T> nl, const T* __restrict__ kx
 #pragma unroll
   for (int f = 0; f < NF; ++f)
 #pragma unroll
-    for (int e = 0; e < E; ++e) nv[f][e] = active ? ld_at(nl.p[f0 + f] + at(e), lane_b) : mk<T>(0, 0);
+    for (int e = 0; e < E; ++e)
+      nv[f][e] = active && iz <= g.keep_z ? ld_at(nl.p[f0 + f] + at(e), lane_b) : mk<T>(0, 0);
   // The x wavenumbers are read from a copy in LDS after the twiddles: loaded from memory per element
   // inside the projection and the update, each was one more wait, and after the first stores a wait
   // for every store in flight as well.
