@@ -1030,13 +1030,14 @@ class Engine : public EngineBase {
   //    256 or 512 rows and there are tiles enough (512^3 3 329 / 6 708 against 3 418 / 6 936, 256^3 435 / 819
   //    against 440 / 834); with 384 or 1024 rows its registers spill into the occupancy (384^3 1 805 / 3 491
   //    against 1 760 / 3 422, 1024 x 128 x 96 516 against 494), and on small grids it waits longer than the
-  //    two launches it replaces (64^3 49 / 54 against 40 / 45).  The colloid has modes 0 to 3, the same two forms
-  //    being 2 and 3 (384 x 256 x 192: 1 133 / 2 038 in mode 2, 1 177 / 2 101 in 3, 1 216 / 2 174 in 1);
+  //    two launches it replaces (64^3 49 / 54 against 40 / 45).  With a colloid the same two forms are modes 2
+  //    and 3 (384 x 256 x 192: 801 / 1 527 in mode 2, 816 / 1 574 in 3, 990 / 1 854 in 1; 512^3 4 943 / 9 006,
+  //    4 849 / 8 819, 6 176 / 11 057);
   //  * fused z pass: FP64 rows of powers of two from 64 on variant 7, whose exchanges are lane swaps from 128 on
   //    (128^2 rows of 64: 24 us against 27 in variant 9, of 128: 41 against 50, of 256: 76 against 88, of 512: 144
   //    against 167); everything else in pairs of rows, 9 or with a colloid 10 (128^2 rows of 96: FP64 62 against
-  //    79, FP32 26 against 51; FP32 rows of 512: 76 against 87; with a colloid FP32 rows of 192 53 against 99, FP64
-  //    114 against 163, but FP64 rows of 256 180 against 101); rows of 1024 have 7 only;
+  //    79, FP32 26 against 51; FP32 rows of 512: 76 against 87; a substage of 128^2 rows of 192 with a
+  //    colloid 156 against 199, FP64 285 against 348, but FP64 rows of 256 396 against 322); rows of 1024 have 7 only;
   //  * standalone z passes persistent in FP32 and on short FP64 rows (512^3 FP32 401 against 456, FP64 820
   //    against 748).
   void default_tuning() {
@@ -1615,8 +1616,9 @@ class Engine : public EngineBase {
   bool lane32() const { return (64LL * ny_ * kzs_ + 64) * (long long)sizeof(C) <= 0xFFFFFFFFLL; }
   // modes 4 and 5: late derivatives (the x pass reads each state field once, the y and z passes
   // apply their own derivatives; see late_inverse), with mode 2's and mode 3's forward side.
-  // Not built for the colloid, whose work fields need second derivatives.
+  // With a colloid modes 2 and 3 have that inverse side already and there are no others.
   int max_xmode() const { return colloid_ ? 3 : 5; }
+  bool late_mode(int mode) const { return mode >= (colloid_ && lane32() ? 2 : 4); }
 
   // Work field w of a substage as an operation on one or two state fields.
   XOp xop_of(int w, const C*& A, const C*& B) const {
@@ -1671,24 +1673,31 @@ class Engine : public EngineBase {
       else xop_launch<L, 8>(ws, n, two, a);
     }
   }
-  // Late-derivative inverse passes (x modes 4, 5).  Work buffers: ws0 u, ws1 v, ws2 w, ws3 w_y,
+  // Late-derivative inverse passes (x modes 4, 5; modes 2 and 3 of a colloid).  Work buffers: ws0 u, ws1 v, ws2 w, ws3 w_y,
   // ws4 w_x, ws5 v_x (then omega_z), per scalar s ws[6+3s] phi_x, ws[7+3s] phi_y, ws[8+3s] phi.
   // The x pass reads u, v, w, phi once each (4 inputs, 4 + 2 + S outputs instead of 12 + 3S
   // inputs and 6 + 3S outputs); the y pass reads 5 + 2S fields and writes 6 + 3S, adding w_y,
   // phi_y and omega_z = v_x - i k_y u; the fused z pass forms omega_x = w_y - i k_z v,
-  // omega_y = i k_z u - w_x and phi_z = i k_z phi as it loads.
+  // omega_y = i k_z u - w_x and phi_z = i k_z phi as it loads.  A colloid adds lap Z (ws[7+3S]) in three
+  // steps: the x pass writes Z_xx, the y pass adds Z_yy, the z pass subtracts k_z^2 Z; c itself is the row c_z is
+  // formed from.  That is 10 outputs of the x pass instead of 14 and 10 inputs of the y pass, 13
+  // outputs instead of 14 (384 x 256 x 192 FP32: x 237 -> 101 us, y 213 -> 197, a substage 911 -> 766; FP64 1732 ->
+  // 1521).
   void late_inverse() {
     if (!lane32()) throw Error(GNSS_ERR_UNSUPPORTED, "late passes address a tile with 32-bit byte offsets");
-    const PairOp copy{1, 1, {1, 0}, {0, 0}, {0, 0}, {0, 0}};        // out0 = A
-    const PairOp copy_d{1, 2, {1, 0}, {0, 1}, {0, 0}, {0, 0}};      // out0 = A, out1 = i k A
-    const PairOp curl_z{2, 2, {1, 0}, {0, -1}, {0, 1}, {0, 0}};     // out0 = A, out1 = B - i k A
+    const PairOp copy{1, {1}, {0}, {0}, {0}};                              // out0 = A
+    const PairOp copy_d{2, {1, 0}, {0, 1}, {0}, {0}};                      // out0 = A, out1 = i k A
+    const PairOp copy_dd{3, {1, 0, 0}, {0, 1, 0}, {0}, {0, 0, 1}};         // and out2 = - k^2 A
+    const PairOp copy_lap{3, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 0, 1}};  // and out2 = B - k^2 A
+    const PairOp curl_z{2, {1, 0}, {0, -1}, {0, 1}, {0}};                  // out0 = A, out1 = B - i k A
     PairList<T> lx{}, ly{};
     int nxe = 0, nye = 0;
-    auto put = [](PairList<T>& l, int& n, const C* A, const C* B, C* o0, C* o1, const PairOp& op) {
+    auto put = [](PairList<T>& l, int& n, const C* A, const C* B, C* o0, C* o1, const PairOp& op, C* o2 = nullptr) {
       l.A[n] = A;
       l.B[n] = B ? B : A;
       l.out[0][n] = o0;
       l.out[1][n] = o1 ? o1 : o0;
+      l.out[2][n] = o2 ? o2 : o0;
       l.op[n] = op;
       ++n;
     };
@@ -1697,7 +1706,8 @@ class Engine : public EngineBase {
     const int CC = pair_chunk(), CY = yc_ ? yc_ : CC;
     const long long xtiles = (long long)kz_tiles(CC) * (2 * g_.keep_y + 1) * bm_ * (3 + S_);
     const bool apart = xtiles * (CC * nx_ / elems_per_thread(nx_)) <= (long long)n_cu_ * 1024;
-    const PairOp deriv{1, 1, {0, 0}, {1, 0}, {0, 0}, {0, 0}};       // out0 = i k A
+    const PairOp deriv{1, {0}, {1}, {0}, {0}};     // out0 = i k A
+    const PairOp deriv2{1, {0}, {0}, {0}, {1}};    // out0 = - k^2 A
     auto put_d = [&](const C* A, C* o0, C* o1) {
       if (apart) {
         put(lx, nxe, A, nullptr, o0, nullptr, copy);
@@ -1709,13 +1719,22 @@ class Engine : public EngineBase {
     put(lx, nxe, q_[0], nullptr, ws_[0], nullptr, copy);
     put_d(q_[1], ws_[1], ws_[5]);
     put_d(q_[2], ws_[2], ws_[4]);
-    for (int q = 0; q < S_; ++q) put_d(q_[3 + q], ws_[8 + 3 * q], ws_[6 + 3 * q]);
+    C* const lap = colloid_ ? ws_[7 + 3 * S_] : nullptr;
+    for (int q = 0; q < S_; ++q) {
+      if (q == 0 && lap && !apart) {
+        put(lx, nxe, q_[3], nullptr, ws_[8], ws_[6], copy_dd, lap);
+      } else {
+        put_d(q_[3 + q], ws_[8 + 3 * q], ws_[6 + 3 * q]);
+        if (q == 0 && lap) put(lx, nxe, q_[3], nullptr, lap, nullptr, deriv2);
+      }
+    }
     put(ly, nye, ws_[0], ws_[5], ws_[0], ws_[5], curl_z);
     put(ly, nye, ws_[1], nullptr, ws_[1], nullptr, copy);
     put(ly, nye, ws_[2], nullptr, ws_[2], ws_[3], copy_d);
     put(ly, nye, ws_[4], nullptr, ws_[4], nullptr, copy);
     for (int q = 0; q < S_; ++q) {
-      put(ly, nye, ws_[8 + 3 * q], nullptr, ws_[8 + 3 * q], ws_[7 + 3 * q], copy_d);
+      if (q == 0 && lap) put(ly, nye, ws_[8], lap, ws_[8], ws_[7], copy_lap, lap);
+      else put(ly, nye, ws_[8 + 3 * q], nullptr, ws_[8 + 3 * q], ws_[7 + 3 * q], copy_d);
       put(ly, nye, ws_[6 + 3 * q], nullptr, ws_[6 + 3 * q], nullptr, copy);
     }
     ColArgs ax;
@@ -1767,7 +1786,7 @@ class Engine : public EngineBase {
     auto rows = [&](int keep) { return keep < 0 ? L : std::min(L, 2 * keep + 1); };
     const double col = (double)a.nouter * a.nchunks * CC * sizeof(C);
     double bytes = 0;
-    for (int i = 0; i < n; ++i) bytes += col * (li.op[i].nin * rows(a.in_keep) + li.op[i].nout * rows(a.out_keep));
+    for (int i = 0; i < n; ++i) bytes += col * ((li.B[i] != li.A[i] ? 2 : 1) * rows(a.in_keep) + li.op[i].nout * rows(a.out_keep));
     timed(name, bytes, [&] {
       switch (L) {
         case 16: pair_c<16>(li, n, a, kv, CC); break;
@@ -1949,7 +1968,7 @@ class Engine : public EngineBase {
     a.S = S_;
     a.colloid = colloid_;
     a.alpha = (T)p_.alpha;
-    a.late = ((p_.flags & GNSS_FLAG_UNFUSED) == 0 && x_mode() >= 4) ? 1 : 0;
+    a.late = ((p_.flags & GNSS_FLAG_UNFUSED) == 0 && late_mode(x_mode())) ? 1 : 0;
     a.kz = tkz_;
     const T scale = (T)(1.0 / ((double)nx_ * ny_ * nz_));
     const double bytes = (double)bm_ * nx_ * ny_ * (double)kz_cols_ * sizeof(C) * (W_ + F_);
@@ -1982,7 +2001,7 @@ class Engine : public EngineBase {
     const int xm = unfused ? 0 : x_mode();
     const bool xf = xm == 1;                  // group-fused inverse side
     const bool xfwd = xm == 1 || xm == 3 || xm == 5;  // group-fused forward side
-    const bool late = xm >= 4;                // late-derivative inverse side
+    const bool late = late_mode(xm);          // late-derivative inverse side
     if (xf) {
       x_fused(true, -1, c);
       for (int q = 0; q < S_; ++q) x_fused(true, q, c);

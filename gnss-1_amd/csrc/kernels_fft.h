@@ -323,6 +323,22 @@ struct ZRow {
     r.nyq = nq ? form(bm, am, kz[M]).x : (T)0;
   }
 
+  // A - kz^2 B (see load_ikz).
+  __device__ __forceinline__ static void load_lap(const cx<T>* __restrict__ A, const cx<T>* __restrict__ B,
+                                                  const T* kzr, const T* __restrict__ kz, bool active, int lim,
+                                                  int t, Raw& r) {
+    Raw b;
+    load(A, active, lim, t, r);
+    load(B, active, lim, t, b);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const T k2 = kzr[e] * kzr[e];
+      r.x[e].x -= k2 * b.x[e].x;
+      r.x[e].y -= k2 * b.x[e].y;
+    }
+    if (M < lim) r.nyq -= kz[M] * kz[M] * b.nyq;
+  }
+
   // Twiddles of one thread for every row it transforms, read once and kept in registers: the
   // radix stages' (TwRegs) and the packing factors twN[k] of its positions k = t + e TPC.  As
   // (E/2) TPC = NZ/4, twN[k] of register e >= E/2 is -i times that of register e - E/2.
@@ -829,8 +845,7 @@ __device__ __forceinline__ void zfused_row(const ZFusedArgs<T>& a, const TM& twM
     // colloidAdvectionKernel_mgpu (solver.cu:374-391): u.grad c + alpha (lap Z c + grad Z . grad c)
     // = (u + alpha grad Z) . grad c + alpha lap Z c, with u + alpha grad Z already in vel.
     const int sc = a.S - 1;
-#pragma unroll
-    for (int b = 0; b < 3; ++b) Z::load(a.ws[6 + 3 * sc + b] + off, active, LIM, t, r0[b]);
+    load_grad(sc);
     Z::template c2r<3, !DEFER>(r0, lds, idx, t, twM, twN, scale, om);  // grad c
     cx<T> n[1][E];
 #pragma unroll
@@ -839,8 +854,13 @@ __device__ __forceinline__ void zfused_row(const ZFusedArgs<T>& a, const TM& twM
       n[0][e] = mk<T>(u.x * om[0][e].x + v.x * om[1][e].x + w.x * om[2][e].x,
                       u.y * om[0][e].y + v.y * om[1][e].y + w.y * om[2][e].y);
     }
+    if (a.late) {
+      Z::load(a.ws[8 + 3 * sc] + off, active, LIM, t, r0[0]);
+      Z::load_lap(a.ws[7 + 3 * a.S] + off, a.ws[8] + off, kzr, a.kz, active, LIM, t, r0[1]);
+    } else {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) Z::load(a.ws[6 + 3 * a.S + b] + off, active, LIM, t, r0[b]);
+      for (int b = 0; b < 2; ++b) Z::load(a.ws[6 + 3 * a.S + b] + off, active, LIM, t, r0[b]);
+    }
     Z::template c2r<2, !DEFER>(r0, lds, idx, t, twM, twN, scale, om);  // c, lap Z
 #pragma unroll
     for (int e = 0; e < E; ++e) fma_pair(n[0][e], mk<T>(a.alpha * om[1][e].x, a.alpha * om[1][e].y), om[0][e]);
@@ -1015,7 +1035,7 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
     H::load(a.ws[w0 + 1] + off, active, LIM, t, r[1]);
     if (a.late) H::template load_ikz<0, 1>(a.ws[w0 + 2] + off, a.ws[w0 + 2] + off, kzr, a.kz, active, LIM, t, r[2]);
     else H::load(a.ws[w0 + 2] + off, active, LIM, t, r[2]);
-    if (col) H::load(a.ws[6 + 3 * a.S] + off, active, LIM, t, r[3]);
+    if (col) H::load(a.ws[a.late ? w0 + 2 : 6 + 3 * a.S] + off, active, LIM, t, r[3]);
     cx<T> zg[2][E];
     Z::pack(r[0], r[1], t, zg[0]);
     if (col) Z::pack(r[2], r[3], t, zg[1]);
@@ -1038,7 +1058,8 @@ __device__ __forceinline__ void zfused_pair_row(const ZFusedArgs<T>& a, const TW
           w[e] += a.alpha * zg[1][e].x;
         }
       } else if (col) {
-        H::load(a.ws[7 + 3 * a.S] + off, active, LIM, t, r[0]);
+        if (a.late) H::load_lap(a.ws[7 + 3 * a.S] + off, a.ws[8] + off, kzr, a.kz, active, LIM, t, r[0]);
+        else H::load(a.ws[7 + 3 * a.S] + off, active, LIM, t, r[0]);
         Z::pack(r[0], zero, t, zb[0]);
         lds_sync<true>();
         fft_batch<T, N, +1, Pad, P, true, 1, RS>(zb, lds, t, idx, tw);

@@ -773,21 +773,21 @@ k_xinv_op_pipe(XOpList<T> li, const T* __restrict__ kxv, const T* __restrict__ k
 }
 
 // Inverse strided passes with the derivatives along the transformed axis applied on the way in
-// (the late-derivative x mode): list entry i reads one or two input fields A, B and writes one or
-// two transformed outputs out_j = (a_j + i b_j k) A + (c_j + i d_j k) B with a_j .. d_j in
-// {-1, 0, 1}, k the wavenumber of the element's mode along the axis.  The x pass reads the state
+// (the late-derivative x mode): list entry i reads one or two input fields A, B and writes one to
+// three transformed outputs out_j = (a_j + i b_j k) A + c_j B, or - d_j k^2 A + c_j B where d_j is not 0, with
+// a_j .. d_j in {-1, 0, 1}, k the wavenumber of the element's mode along the axis.  The x pass reads the state
 // once per field (u, v, w, phi) and writes it with its x-derivatives; the y pass adds the
 // y-derivatives and omega_z = v_x - i k_y u; the fused z pass forms the remaining terms with
 // i k_z (replaces the spectral prologue of the reference's computeRHS, solver.cu:419-437, and the
 // curl/gradient kernels it calls).
 struct PairOp {
-  int nin, nout;
-  float a[2], b[2], c[2], d[2];
+  int nout;
+  float a[3], b[3], c[3], d[3];
 };
 template <typename T> struct PairList {
   const cx<T>* A[MAXW];
   const cx<T>* B[MAXW];
-  cx<T>* out[2][MAXW];
+  cx<T>* out[3][MAXW];
   PairOp op[MAXW];
 };
 
@@ -816,7 +816,7 @@ constexpr unsigned removed_slabs(int L, int TPC, int E) {
 // 334 -> 276.)  Columns of removed modes end at once and only rows inside the ellipsoid are loaded.
 // The twiddles and the axis' wavenumbers are read from copies in LDS, after the data regions.  An entry
 // may write its outputs over its own inputs (the block that owns a tile writes output 0 last, over input
-// A, and output 1 only after reading B); no entry may read a field another entry writes.
+// A, and the last output, the only one to take B, over B); no entry may read a field another entry writes.
 template <typename T, int L, int C>
 __global__ void __launch_bounds__(lb_threads(C * (L / ColPlan<T, L>::E)), (col_waves<T, L, C>()))
 k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ tw, ColArgs a, int tpf) {
@@ -862,18 +862,26 @@ k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ t
                  ? ld_at(src + off + (long long)e * TPC * a.estride, lane_b)
                  : mk<T>(0, 0);
   };
-  // the second output first: the first may be written over the inputs
+  // the last output first: the first may be written over the inputs
 #pragma unroll 1
   for (int j = li.op[ent].nout - 1; j >= 0; --j) {
     const PairOp* op = &li.op[ent];
-    const T ra = (T)(j ? op->a[1] : op->a[0]), ba = (T)(j ? op->b[1] : op->b[0]), rb = (T)(j ? op->c[1] : op->c[0]);
+    const T ra = (T)op->a[j], ba = (T)op->b[j], rb = (T)op->c[j], da = (T)op->d[j];
     cx<T> v[1][E];
     load(li.A[ent], v[0]);
     __syncthreads();  // the copies are there, and the LDS of the last transform is free
+    if (da != (T)0) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const T ka = ba * kl[t + e * TPC];
-      v[0][e] = mk<T>(ra * v[0][e].x - ka * v[0][e].y, ra * v[0][e].y + ka * v[0][e].x);
+      for (int e = 0; e < E; ++e) {
+        const T k = kl[t + e * TPC], k2 = -da * k * k;
+        v[0][e] = mk<T>(k2 * v[0][e].x, k2 * v[0][e].y);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const T ka = ba * kl[t + e * TPC];
+        v[0][e] = mk<T>(ra * v[0][e].x - ka * v[0][e].y, ra * v[0][e].y + ka * v[0][e].x);
+      }
     }
     if (rb != (T)0) {
       cx<T> vb[E];
@@ -886,7 +894,7 @@ k_inv_late(PairList<T> li, const T* __restrict__ kv, const cx<T>* __restrict__ t
     }
     fft_batch<T, L, +1, LdsCol, P, false, 1, L * C>(v, lds, t, idx, twl);
     if (r.live) {
-      cx<T>* __restrict__ dst = j ? li.out[1][ent] : li.out[0][ent];
+      cx<T>* __restrict__ dst = li.out[j][ent];
 #pragma unroll
       for (int e = 0; e < E; ++e) st_at(dst + off + (long long)e * TPC * a.estride, lane_b, v[0][e]);
     }
