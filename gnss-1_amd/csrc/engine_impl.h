@@ -620,12 +620,8 @@ class Engine : public EngineBase {
       const long long nm = (long long)b.bx * b.by * b.bz;
       hipLaunchKernelGGL(k_vorticity<T>, dim3((unsigned)cdiv(nm, 256)), dim3(256), 0, s_, g_, b, ptrs(q_), w, tkx_,
                          tky_, tkz_, nm);
-      T* om[3];
-      for (int c = 0; c < 3; ++c) om[c] = reinterpret_cast<T*>(ws_[3 + c]);
-      inv3d(ws_.data(), ws_.data(), om, 3, clean_);
       out = reinterpret_cast<T*>(ws_[3]);
-      hipLaunchKernelGGL(k_magnitude<T>, dim3((unsigned)cdiv(nph_, 256)), dim3(256), 0, s_, out,
-                         reinterpret_cast<const T*>(ws_[4]), reinterpret_cast<const T*>(ws_[5]), nph_);
+      z_c2r_length(ws_.data(), out, inv_xy(ws_.data(), ws_.data(), 3, clean_));
     }
     GNSS_HIP(hipGetLastError());
     return out;
@@ -1482,6 +1478,19 @@ class Engine : public EngineBase {
     return per_cu * n_cu_;
   }
 
+  template <int NZ>
+  void zlength_launch(const ZList<T>& zl, int in_lim) {
+    constexpr int M = NZ / 2;
+    using FP = FusedPlan<T, M, 3>;
+    constexpr int TPC = M / FP::type::E;
+    const long long row_lds = (long long)FUSED_B * FP::pad::stride(M) * (long long)sizeof(C);
+    int G = std::max(1, 256 / TPC);
+    while (G > 1 && G * row_lds > LDS_MAX) --G;
+    const long long rows = (long long)nx_ * ny_;
+    hipLaunchKernelGGL((k_c2r_length<T, NZ>), dim3((unsigned)cdiv(rows, G)), dim3(TPC * G), (size_t)(G * row_lds), s_, zl,
+                       tw_.at(M), tw_.at(NZ), rows, kzs_, in_lim, (T)(1.0 / ((double)nx_ * ny_ * nz_)), G);
+  }
+
 #define GNSS_Z_SWITCH(FN, ...)                                                                 \
   switch (nz_) {                                                                               \
     case 16: FN<16>(__VA_ARGS__); break;                                                       \
@@ -1499,6 +1508,13 @@ class Engine : public EngineBase {
     default: throw Error(GNSS_ERR_UNSUPPORTED, "unsupported nz " + std::to_string(nz_));      \
   }
 
+  void z_c2r_length(const C* const* in, T* out, int lim) {
+    ZList<T> zl{};
+    for (int c = 0; c < 3; ++c) zl.in[c] = in[c];
+    zl.out[0] = out;
+    const double bytes = (double)nx_ * ny_ * ((double)nz_ * sizeof(T) + 3.0 * std::min(lim, nzh_) * sizeof(C));
+    timed("fft_z_c2r_length", bytes, [&] { GNSS_Z_SWITCH(zlength_launch, zl, lim); });
+  }
   void z_r2c(const T* in, C* out, int out_lim) {
     const double bytes = (double)nx_ * ny_ * ((double)nz_ * sizeof(T) + (double)std::min(out_lim, kzs_) * sizeof(C));
     timed("fft_z_r2c", bytes, [&] { GNSS_Z_SWITCH(zr2c_launch, in, out, out_lim); });
@@ -1535,16 +1551,18 @@ class Engine : public EngineBase {
   // and writes another is cheaper along y (512^3 FP32: 0.19 ms) than along x, where every row of a tile
   // is a page of its own in both (0.30 ms, 0.23 ms in place).
   void inv3d(const C* const* spec, C* const* work, T* const* out, int nf, bool prune) {
-    const T scale = (T)(1.0 / ((double)nx_ * ny_ * nz_));
+    z_c2r(work, out, nf, inv_xy(spec, work, nf, prune), (T)(1.0 / ((double)nx_ * ny_ * nz_)));
+  }
+  // its strided passes; returns the length of the rows they leave
+  int inv_xy(const C* const* spec, C* const* work, int nf, bool prune) {
     if (!prune) {
       col_passes(spec, work, nf, ColSpec{1, +1, kzs_ / cy_, -1, -1, -1});
       col_passes(work, nf, ColSpec{0, +1, kzs_ / cx_, -1, -1, -1});
-      z_c2r(work, out, nf, nzh_, scale);
-      return;
+      return nzh_;
     }
     col_passes(spec, work, nf, ColSpec{0, +1, kz_lim_ / cx_, g_.keep_y, g_.keep_x, -1});
     col_passes(work, nf, ColSpec{1, +1, kz_lim_ / cy_, -1, g_.keep_y, -1});
-    z_c2r(work, out, nf, kz_lim_, scale);
+    return kz_lim_;
   }
   void inv3d(C* spec, T* out, bool prune) { inv3d(&spec, &spec, &out, 1, prune); }
   // the state's fields f0 .. f0 + nf - 1, left as they are

@@ -1172,15 +1172,6 @@ __global__ void k_vorticity(Geom g, Box b, CPtrs<T> q, CPtrs<T> w, const T* __re
   w.p[2][o] = csub(ik(kx, v), ik(ky, u));
 }
 
-// |(a, b, c)| in place over a (VectorMagnitude_kernel, statistics.cu:2005-2018).
-template <typename T>
-__global__ void k_magnitude(T* __restrict__ a, const T* __restrict__ b, const T* __restrict__ c, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T x = a[i], y = b[i], z = c[i];
-  a[i] = sqrt(x * x + y * y + z * z);
-}
-
 // One physical plane of [x][y][z]: axis 2 (z = index) -> [x][y], axis 1 -> [x][z],
 // axis 0 -> [y][z] (writexyfields / writexzfields / writeyzfields, iofuncs.cu:187-260).
 template <typename T>
