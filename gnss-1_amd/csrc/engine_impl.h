@@ -519,15 +519,18 @@ class Engine : public EngineBase {
     GNSS_HIP(hipEventCreate(&e0));
     GNSS_HIP(hipEventCreate(&e1));
     GNSS_HIP(hipEventCreate(&e2));
-    // warm-up pair
-    const C* spec = q_[0];
-    inv3d(&spec, ws_.data(), phys_.data(), 1, false);
+    // warm-up pair; the inverse is timed in place, on a copy of the state
+    auto inverse = [&] {
+      GNSS_HIP(hipMemcpyAsync(ws_[0], q_[0], sizeof(C) * nsp_, hipMemcpyDeviceToDevice, s_));
+      GNSS_HIP(hipEventRecord(e1, s_));
+      inv3d(ws_[0], phys_[0], false);
+      GNSS_HIP(hipEventRecord(e2, s_));
+    };
+    inverse();
     fwd3d(phys_[0], ws_[1], false);
     float tf = 0, ti = 0;
     for (int r = 0; r < reps; ++r) {
-      GNSS_HIP(hipEventRecord(e1, s_));
-      inv3d(&spec, ws_.data(), phys_.data(), 1, false);
-      GNSS_HIP(hipEventRecord(e2, s_));
+      inverse();
       GNSS_HIP(hipEventSynchronize(e2));
       float a = 0, b = 0;
       GNSS_HIP(hipEventElapsedTime(&a, e1, e2));
@@ -1260,11 +1263,13 @@ class Engine : public EngineBase {
   void col_launch(const FieldList<T>& fl, int nf, const ColArgs& a, int G, int axis) {
     // both forms hold the twiddle table in LDS, after the data regions
     const size_t lds = ((size_t)G * L * CC + L) * sizeof(C);
-    // Persistent for x passes with cp only: their rows lie a page apart, and one block that loads ahead has
-    // fewer of them open (512^3, whole arrays: FP32 0.24 against 0.25 ms, FP64 0.48 against 0.51); along y
-    // two blocks per CU win at every size (forward pass of a substage at 512^3: FP32 0.43 against 0.48 ms,
-    // FP64 0.85 against 0.88; at 256^3 0.057 against 0.068 and 0.119 against 0.145).
-    if (cp_ && axis == 0) {
+    // Persistent for x passes with cp and for whole arrays well beyond the last-level cache: their rows lie a page
+    // apart, and one block that loads ahead has fewer of them open (512^3 FP32 0.239 against 0.251 ms, FP64 0.477
+    // against 0.511; 384^3 FP64 192 against 211 us, 256 x 512 x 512 FP64 216 against 234; below, 384 x 512 x 512
+    // FP32 of 428 MB 195 against 157, 256^3 FP64 59 against 54).  Pruned x passes (512^3 FP32 97 against 80 us) and,
+    // at every size, y passes (forward pass of a substage at 512^3 FP32 0.48 against 0.43 ms) have two blocks per CU.
+    const bool whole = a.in_keep < 0 && a.out_keep < 0 && a.outer_keep < 0;
+    if (axis == 0 && (cp_ || (whole && nsp_ * (long long)sizeof(C) > (448LL << 20)))) {
       constexpr int TPC = L / Plan<L>::E;
       const int threads = CC * TPC * G;
       const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
