@@ -882,8 +882,8 @@ class Engine : public EngineBase {
   // A batched context's own entry ("<key>b"): its launches cover every member, so other pass
   // variants can win than for one member of the grid.  Batched steps always run the late x mode;
   // the fused z variant is timed alone, then the inverse passes' tile jointly with persistent or
-  // per-tile column passes (cp), one launch per pass or per field (cb) and the late passes' output
-  // form (lp), then the forward passes' tiles (cx, cy) and the late y passes' own tile (yc) — all
+  // per-tile column passes (cp), one launch per pass or per field (cb) and lp (of which the late
+  // passes have one form left: its candidates repeat), then the forward passes' tiles (cx, cy) and the late y passes' own tile (yc) — all
   // over whole middle substages of every member, on a snapshot of the state restored afterwards.
   std::string autotune_batched(int reps) {
     const std::string key = tuning_key() + "b";

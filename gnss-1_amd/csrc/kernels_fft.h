@@ -763,7 +763,7 @@ __device__ __forceinline__ void zfused_row(const ZFusedArgs<T>& a, const TM& twM
   constexpr bool DEFER = FP::defer;
   const T h = DEFER ? (T)0.5 * scale * scale : (T)0.5;
   // the pruned row length is the same for every launch of a grid (kz below the 2/3 rule, rounded up
-  // to the widest column tile): as a constant it lets the compiler drop the loads, shuffles and
+  // to 64 bytes): as a constant it lets the compiler drop the loads, shuffles and
   // packing of the entries known to be zero and the unpacking of the entries never stored
   constexpr int LIM = zfused_lim<T>(NZ);
   const long long row = (long long)blockIdx.x * a.G + g;

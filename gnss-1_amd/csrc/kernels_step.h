@@ -807,8 +807,8 @@ constexpr unsigned removed_slabs(int L, int TPC, int E) {
 }
 
 // One block per tile, over the entries of a whole pass: tile i is tile i % tpf of list entry i / tpf, entries
-// of one or two inputs and outputs together (the branches are uniform over the block), so a pass is one
-// launch.  Two outputs go through the radix stages one after the other in one LDS region, each from a
+// of one or two inputs and one to three outputs together (the branches are uniform over the block), so a pass is one
+// launch.  The outputs go through the radix stages one after the other in one LDS region, each from a
 // load of its own: the inputs stay in the L2, and a block keeps one set of values, which leaves room
 // for two blocks per CU whose transforms and memory phases overlap.  (As one persistent block per CU
 // that loaded the next tile ahead, its barriers put every wave into the same phase: 512^3 FP32 x 525 and
