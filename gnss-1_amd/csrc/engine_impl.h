@@ -1266,10 +1266,11 @@ class Engine : public EngineBase {
     // Persistent for x passes with cp and for whole arrays well beyond the last-level cache: their rows lie a page
     // apart, and one block that loads ahead has fewer of them open (512^3 FP32 0.239 against 0.251 ms, FP64 0.477
     // against 0.511; 384^3 FP64 192 against 211 us, 256 x 512 x 512 FP64 216 against 234; below, 384 x 512 x 512
-    // FP32 of 428 MB 195 against 157, 256^3 FP64 59 against 54).  Pruned x passes (512^3 FP32 97 against 80 us) and,
+    // FP32 of 428 MB 195 against 157, 256^3 FP64 59 against 54; 1024 rows, whose tiles are whole lines, 307 against
+    // 257 at 1024 x 256 x 256 FP64).  Pruned x passes (512^3 FP32 97 against 80 us) and,
     // at every size, y passes (forward pass of a substage at 512^3 FP32 0.48 against 0.43 ms) have two blocks per CU.
     const bool whole = a.in_keep < 0 && a.out_keep < 0 && a.outer_keep < 0;
-    if (axis == 0 && (cp_ || (whole && nsp_ * (long long)sizeof(C) > (448LL << 20)))) {
+    if (axis == 0 && (cp_ || (whole && L < 1024 && nsp_ * (long long)sizeof(C) > (448LL << 20)))) {
       constexpr int TPC = L / Plan<L>::E;
       const int threads = CC * TPC * G;
       const long long blocks = (long long)a.nchunks * cdiv(a.nouter, G);
@@ -1365,7 +1366,8 @@ class Engine : public EngineBase {
   void col_passes(C* const* fields, int nf, const ColSpec& sp) { col_passes(fields, fields, nf, sp); }
   void col_passes(const C* const* in, C* const* fields, int nf, const ColSpec& sp) {
     const int L = sp.axis == 0 ? nx_ : ny_;
-    const int CC = sp.axis == 0 ? cx_ : cy_;
+    const int given = sp.axis == 0 ? cx_ : cy_;
+    const int CC = F64 || sp.axis == 0 || !sp.pruned() ? full_lines(L, given) : given;
     const int TPC = L / elems_per_thread(L);
     ColArgs a;
     if (sp.axis == 1) {
@@ -1381,10 +1383,11 @@ class Engine : public EngineBase {
       a.outer_n = ny_;
       a.nouter = sp.outer_keep < 0 ? ny_ : 2 * sp.outer_keep + 1;
     }
-    a.nchunks = sp.nchunks;
+    const int cols = sp.nchunks * given;
+    a.nchunks = (cols + CC - 1) / CC;
     a.in_keep = sp.in_keep;
     a.out_keep = sp.out_keep;
-    a.cols = sp.cols ? sp.cols : sp.nchunks * CC;
+    a.cols = sp.cols ? sp.cols : cols;
     if (sp.pruned()) a.sph = sphere(sp.axis);
     batch_outer(a);
     int G = std::max(1, 256 / (CC * TPC));
@@ -1726,7 +1729,7 @@ class Engine : public EngineBase {
     };
     // Small grids take a field and its x derivative in blocks of their own (the passes' outputs are not their
     // inputs): the launch then lasts one transform instead of two.
-    const int CC = pair_chunk(), CY = yc_ ? yc_ : CC;
+    const int CC = full_lines(nx_, xc_), CY = yc_ ? yc_ : xc_;
     const long long xtiles = (long long)kz_tiles(CC) * (2 * g_.keep_y + 1) * bm_ * (3 + S_);
     const bool apart = xtiles * (CC * nx_ / elems_per_thread(nx_)) <= (long long)n_cu_ * 1024;
     const PairOp deriv{1, {0}, {1}, {0}, {0}};     // out0 = i k A
@@ -1789,7 +1792,16 @@ class Engine : public EngineBase {
     pair_pass(lx, nxe, ax, nx_, tkx_, "fft_x_inv_late", CC);
     pair_pass(ly, nye, ay, ny_, tky_, "fft_y_inv_late", CY);
   }
-  int pair_chunk() const { return xc_; }
+  // Passes of 1024 rows are given tiles of half a memory line (64 bytes: LDS_MAX for two blocks per CU); a tile of
+  // whole lines in one block per CU is faster along x, where a line is all that a row's page gives (1024 x 256 x
+  // 256, late x pass FP32 325 -> 271 us, FP64 673 -> 441; whole forward x FP32 203 -> 135, FP64 353 -> 257; 1024 x
+  // 512 x 512, substage FP32 7.36 -> 6.94 ms, FP64 14.5 -> 13.3), in whole passes along y
+  // (128 x 1024 x 96 FP32 47 -> 33) and in FP64 along y (124 -> 118), but not in FP32's pruned forward y pass (73
+  // against 78), nor does the late y pass gain (149 either way).
+  static constexpr bool F64 = sizeof(T) == 8;
+  int full_lines(int L, int c) const {
+    return L == 1024 && c * (int)sizeof(C) == 64 && !(p_.flags & GNSS_FLAG_MFMA_R16) ? 2 * c : c;
+  }
   int kz_tiles(int cc) const { return (kz_cols_ + cc - 1) / cc; }  // column tiles of a substage's passes
   // The 2/3 rule's ellipsoid for a pruned pass over kx (axis 0) or ky (1) rows.  Off for the MFMA
   // passes, which read and write whole boxes.
